@@ -2,6 +2,7 @@
 // gemm_kernel.h).  Built without the VGPR-form MFMA option that gemm.hip
 // uses: each wavefront holds 128x128 fp32 accumulators (256 per lane), which
 // need the AGPRs; forced into VGPRs they cost 5-7% at M = 4096.
+#define KBN_ACC_AGPR 1
 #include "gemm_kernel.h"
 
 namespace kbn {

@@ -34,6 +34,8 @@
 #include "kbn_common.h"
 
 #include <algorithm>
+#include <type_traits>
+#include <utility>
 
 namespace kbn {
 
@@ -47,7 +49,16 @@ typedef float v16f __attribute__((ext_vector_type(16)));
 // significand in [1, 2).  Zero and subnormal scales get byte 0 (2^-127), so
 // their block adds at most 2^-127 of the value it would have at scale 1;
 // inf/NaN scales get 255, the E8M0 NaN.
-__device__ __forceinline__ int scale_exp_byte(float s) { return (int)((__float_as_uint(s) >> 23) & 0xFFu); }
+// The block-scaled MFMA takes the byte its op_sel names, here the top one:
+// the exponent field lands there with one shift.
+__device__ __forceinline__ int scale_exp_top(float s) { return (int)(__float_as_uint(s) << 1); }
+// UE8M0 contract: the exponent field of s, one more where a mantissa bit is
+// set (s rounded up to a power of two), at most 254, in the top byte: the
+// shift drops the sign, the add carries into the exponent.
+__device__ __forceinline__ int ue8m0_ceil_top(float s) {
+    const uint32_t u = __float_as_uint(s) << 1;
+    return (int)((u < 0xFE000000u ? u : 0xFE000000u) + 0x00FFFFFFu);
+}
 __device__ __forceinline__ float scale_mant(float s) {
     return __uint_as_float((__float_as_uint(s) & 0x007FFFFFu) | 0x3F800000u);
 }
@@ -129,32 +140,74 @@ __device__ __forceinline__ v4i make_desc(const void* base, int64_t bytes) {
     const uint64_t p = reinterpret_cast<uint64_t>(base);
     const uint32_t n = bytes <= 0 ? 0u : (bytes >= 0xFFFFFFFFLL ? 0xFFFFFFFFu : (uint32_t)bytes);
     v4i r;
-    r[0] = (int)(uint32_t)p;
-    r[1] = (int)((p >> 32) & 0xFFFFu);
-    r[2] = (int)n;
+    r[0] = __builtin_amdgcn_readfirstlane((int)(uint32_t)p);
+    r[1] = __builtin_amdgcn_readfirstlane((int)((p >> 32) & 0xFFFFu));
+    r[2] = __builtin_amdgcn_readfirstlane((int)n);
     r[3] = (int)kRsrcWord3;
     return r;
 }
 
 // Direct global->LDS DMA.  Issued as inline asm so the compiler's waitcnt
 // pass does not serialise every LDS read behind the in-flight DMA of the
-// other stage; completion is awaited explicitly (wait_dma) before the
-// barrier that publishes a stage.  Lane i writes LDS bytes
-// [lds + 16*i, lds + 16*i + 16) (dwordx4) or [lds + 4*i, lds + 4*i + 4) (dword).
-__device__ __forceinline__ void dma_b128(const v4i& desc, uint32_t lds, int voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(desc)
-                 : "memory");
+// other stages; completion is awaited explicitly (wait_dma_n) before the
+// barrier that publishes a stage.  Lane i writes LDS bytes [lds + 16 i, +16)
+// (b128) or [lds + 4 i, +4) (b32), lds = base + kOff; it reads the buffer at
+// voff + soff, and the range check covers it whether or not the hardware
+// counts soff (every offset that must read zeros is out of range by voff
+// alone, and soff never exceeds the range).
+// The pair fills lds and lds + 1024 from v0 and v1: one M0 write for two
+// loads, the second through the instruction offset, which moves both
+// addresses, so v1 is the row's offset less 1024 (never negative: its row is
+// at least 8 rows of 128 bytes in).  kNt: the weight rows of a tile are read
+// once per workgroup and should not push the activation rows (read by every
+// workgroup of a tile row) out of L2.
+template <int kOff>
+__device__ __forceinline__ void dma_b32(const v4i& desc, uint32_t base, int voff, int soff) {
+    asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dword %2, %3, %4 offen lds" ::"s"(base), "n"(kOff), "v"(voff),
+                 "s"(desc), "s"(soff)
+                 : "memory", "scc");
 }
-// The same load with the non-temporal hint: the weight rows of a tile are
-// read once per workgroup and should not push the activation rows (read by
-// every workgroup of a tile row) out of L2.
-__device__ __forceinline__ void dma_b128_nt(const v4i& desc, uint32_t lds, int voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dwordx4 %1, %2, 0 offen nt lds" ::"s"(lds), "v"(voff), "s"(desc)
-                 : "memory");
+template <int kOff, bool kNt>
+__device__ __forceinline__ void dma_b128(const v4i& desc, uint32_t base, int voff, int soff) {
+    if constexpr (kNt)
+        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds" ::"s"(base), "n"(kOff),
+                     "v"(voff), "s"(desc), "s"(soff)
+                     : "memory", "scc");
+    else
+        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" ::"s"(base), "n"(kOff),
+                     "v"(voff), "s"(desc), "s"(soff)
+                     : "memory", "scc");
 }
-__device__ __forceinline__ void dma_b32(const v4i& desc, uint32_t lds, int voff) {
-    asm volatile("s_mov_b32 m0, %0\n\tbuffer_load_dword %1, %2, 0 offen lds" ::"s"(lds), "v"(voff), "s"(desc)
-                 : "memory");
+template <int kOff, bool kNt>
+__device__ __forceinline__ void dma_b128_pair(const v4i& desc, uint32_t base, int v0, int v1, int soff) {
+    if constexpr (kNt)
+        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %4, %5 offen nt lds\n\t"
+                     "buffer_load_dwordx4 %3, %4, %5 offen offset:1024 nt lds" ::"s"(base),
+                     "n"(kOff), "v"(v0), "v"(v1), "s"(desc), "s"(soff)
+                     : "memory", "scc");
+    else
+        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
+                     "buffer_load_dwordx4 %3, %4, %5 offen offset:1024 lds" ::"s"(base),
+                     "n"(kOff), "v"(v0), "v"(v1), "s"(desc), "s"(soff)
+                     : "memory", "scc");
+}
+// No instruction, but a volatile use of a value: the MFMA that makes it stays
+// before this point.  MFMAs have no side effects, and without this the
+// compiler sinks those of a K block's first half behind the block's barrier
+// (256x256 tiles 7% slower).  kAgpr: the accumulators live in AGPRs.
+template <bool kAgpr>
+__device__ __forceinline__ void keep_here(float x) {
+    if constexpr (kAgpr) asm volatile("" ::"a"(x));
+    else asm volatile("" ::"v"(x));
+}
+// f(integral_constant<int, 0>), ..., f(integral_constant<int, N - 1>)
+template <class F, int... I>
+__device__ __forceinline__ void static_for_seq(F&& f, std::integer_sequence<int, I...>) {
+    (f(std::integral_constant<int, I>{}), ...);
+}
+template <int N, class F>
+__device__ __forceinline__ void static_for(F&& f) {
+    static_for_seq(f, std::make_integer_sequence<int, N>{});
 }
 __device__ __forceinline__ void wait_dma() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 // Wait until at most N vector-memory loads of this wavefront are outstanding
@@ -350,8 +403,10 @@ constexpr int gemm_occupancy(int bm, int bn, int stages, int fuse_a = 0) {
 // Block-scaled GEMM tile kernel: BM x BN output tile, four wavefronts in a
 // 2 x 2 grid, each owning a (BM/2) x (BN/2) block of 32x32 MFMA fragments.
 //
-// LDS stage layout (one stage = one 128-K block):
-//   [A: BM x 128 B][W: BN x 128 B][sA: 4 x 64 fp32][sW: 4 x 64 fp32]
+// LDS layout, operand by operand (one stage = one 128-K block):
+//   kStages x [A: BM x 128 B], kStages x [W: BN x 128 B], kStages x [sA: 4 x 64 fp32][sW: 4 x 64 fp32]
+// so that every fragment read of every stage is one per-lane base register
+// plus an instruction offset (16 bits).
 // Every load is a 16-B (or 4-B) direct global->LDS DMA; one A/W instruction
 // moves eight full 128-B rows, so every request the vector cache sends to L2
 // is a whole 128-B line.
@@ -410,7 +465,7 @@ gemm_bs_kernel(const GemmArgs a) {
     constexpr int kA = gemm_a_stage_bytes(BM, kFuseA), kB = BN * kRowB, kSA = kWaves * 256, kSW = kWaves * 256;
     constexpr int kAW = 4 * (kFuseA ? kFuseA : 1);     // fused A: LDS rows per wavefront
     constexpr int kStage = kA + kB + kSA + kSW;
-    static_assert(kStages >= 2 && kStages * kStage <= 160 * 1024, "LDS budget");
+    static_assert(kStages >= 2 && kStages <= 4 && kStages * kStage <= 160 * 1024, "LDS budget");
     __shared__ __attribute__((aligned(1024))) uint8_t smem[kStages * kStage];
     const uint32_t lds0 = (uint32_t)reinterpret_cast<uintptr_t>((__attribute__((address_space(3))) uint8_t*)smem);
 
@@ -461,10 +516,10 @@ gemm_bs_kernel(const GemmArgs a) {
         return (t >= 0 && t < a.num_valid) ? t : -1;
     };
 
-    const v4i dA = kFuseA  ? make_desc(a.X + (int64_t)m0 * a.ldx, ((int64_t)(a.M - m0 - 1) * a.ldx + a.K) * 2)
+    v4i dA = kFuseA  ? make_desc(a.X + (int64_t)m0 * a.ldx, ((int64_t)(a.M - m0 - 1) * a.ldx + a.K) * 2)
                    : kSorted ? make_desc(a.A, a.A_bytes)
                              : make_desc(a.A + (int64_t)m0 * a.lda, (int64_t)(a.M - m0 - 1) * a.lda + a.K);
-    const v4i dW = make_desc(Wbase + (int64_t)n0 * a.ldw, (int64_t)(a.N - n0 - 1) * a.ldw + a.K);
+    v4i dW = make_desc(Wbase + (int64_t)n0 * a.ldw, (int64_t)(a.N - n0 - 1) * a.ldw + a.K);
     const v4i dSA = make_desc(a.sA, a.sA_bytes);
     const v4i dSW = kRowW ? make_desc(a.sWp, a.sWp_bytes) : make_desc(sWbase, (int64_t)NB * a.sW_ld * 4);
 
@@ -530,21 +585,20 @@ gemm_bs_kernel(const GemmArgs a) {
         }
     }
     const bool sa_live = sa_src >= 0;
-    const int sa_kstep = sa_live ? (int)(a.sA_sk * 4) : 0;
+    const int sa_kstep = (int)(a.sA_sk * 4);
     const int sa_off0 = sa_live ? (int)((int64_t)sa_src * a.sA_sm * 4) + kb0 * sa_kstep : kOob;
     // W scales of a stage: the tile's 128-row block scales (lane < BN / 128),
     // or with kRowW one packed word per tile row (row wave * 64 + lane): its
     // four K blocks' exponents, word (kb / 4) of the row
-    int sw_kstep, sw_off0;
+    const int sw_kstep = kRowW ? (int)(a.sWp_sk * 4) : 4;
+    int sw_off0;
     if constexpr (kRowW) {
         const int r = wave * 64 + lane;
         const bool live = r < BN && n0 + r < a.N;
-        sw_kstep = live ? (int)(a.sWp_sk * 4) : 0;
         sw_off0 = live ? (int)((int64_t)(n0 + r) * a.sWp_sn * 4) : kOob;
     } else {
         // the scale blocks the tile's rows touch (a 192-row tile may start mid-block)
         const bool sw_live = kGlu ? lane < 2 : (lane < (((n0 & 127) + BN + 127) >> 7)) & (n0 / 128 + lane < NB);
-        sw_kstep = sw_live ? 4 : 0;
         // kGlu: the gate block, then the up block
         const int sw_blk = kGlu ? (lane == 0 ? n0 : a.glu_half + n0) / 128 : n0 / 128 + lane;
         sw_off0 = sw_live ? sw_blk * (int)a.sW_ld * 4 + kb0 * 4 : kOob;
@@ -557,34 +611,85 @@ gemm_bs_kernel(const GemmArgs a) {
     // which measures faster where A and W tiles are both re-read from L2.
     constexpr bool kWeightNt = (BN == 128) || kGrouped || kSorted;
 
-    // DMA instruction d (0 <= d < kDma) of K block s -> LDS buffer s % kStages:
-    // the two scale vectors, then the A rows, then the W rows.  `live` false
-    // turns the load into an out-of-range (zero) read, so the loop never
-    // branches around it and every stage issues the same number of loads.
-    auto issue_one = [&](int s, bool live, int d) {
-        const uint32_t base = lds0 + (s % kStages) * kStage;
-        const int k0 = s * kRowB;
-        if (!kFuseA && d == 0) {
-            dma_b32(dSA, base + kA + kB + wave * 256, live ? sa_off0 + s * sa_kstep : kOob);
-        } else if (d == kScaleDma - 1) {
-            if constexpr (kRowW)
-                dma_b32(dSW, base + kA + kB + kSA + wave * 256, live ? sw_off0 + ((kb0 + s) >> 2) * sw_kstep : kOob);
+    // LDS regions (see the layout above) and this wavefront's part of each
+    constexpr int kOffW = kStages * kA, kOffS = kOffW + kStages * kB;
+    const uint32_t lds_a = lds0 + wave * (kAInstr * 1024), lds_w = lds0 + wave * (kBInstr * 1024),
+                   lds_s = lds0 + wave * 256;
+    // The byte offsets of this lane's loads are fixed for the whole K loop;
+    // the K position enters through the scalar offset.  They stay in
+    // registers where there are few of them; the 256-row tiles add the row
+    // part (uniform) to the first row's offset as each load is issued.
+    // A and W loads go out in pairs that share one M0 write (dma_b128_pair);
+    // gathered rows may lie at offset 0, so they are loaded one by one.
+    constexpr bool kPairW = FM * FN < 8, kPairA = kPairW && !kSorted && kAInstr % 2 == 0;
+    constexpr int kAUnits = kPairA ? kAInstr / 2 : kAInstr, kUnits = kScaleDma + kAUnits + kBInstr / (kPairW ? 2 : 1);
+    constexpr bool kKeepOff = kAInstr + kBInstr <= 12 && FM * FN * kWaves <= 32;
+    auto a_voff = [&](int i) -> int {
+        int off;
+        if constexpr (kFuseA) off = xa_off[i];
+        else if constexpr (kSorted) off = a_row[i] + ((i & 1) ? ch_o : ch_e);
+        else off = ((i & 1) ? a_o : a_e) + (int)(i * 8 * a.lda);
+        if (kPairA && (i & 1)) off -= 1024;
+        if constexpr (kGrouped) off = (a_dead >> i) & 1u ? kOob : off;
+        return off;
+    };
+    auto w_voff = [&](int i) -> int {
+        return ((i & 1) ? (kPairW ? w_o - 1024 : w_o) : w_e) + (int)(i * 8 * a.ldw);
+    };
+    int va[kKeepOff || kGrouped ? kAInstr : 1], vw[kKeepOff ? kBInstr : 1];
+    if constexpr (kKeepOff || kGrouped) {
+#pragma unroll
+        for (int i = 0; i < kAInstr; ++i) va[i] = a_voff(i);
+    }
+    if constexpr (kKeepOff) {
+#pragma unroll
+        for (int i = 0; i < kBInstr; ++i) vw[i] = w_voff(i);
+    }
+    auto a_off = [&](int i) -> int { if constexpr (kKeepOff || kGrouped) return va[i]; else return a_voff(i); };
+    auto w_off = [&](int i) -> int { if constexpr (kKeepOff) return vw[i]; else return w_voff(i); };
+    int s_fetch = 0;   // the block to fetch next (0, with A and W unreadable, past the last)
+    // Load unit u (0 <= u < kUnits) of the block to fetch next, into stage S
+    // (a constant where the stages are unrolled): the scale vectors, then the
+    // A rows, then the W rows.
+    auto issue_unit = [&](auto S_, auto u_) {
+        constexpr int u = decltype(u_)::value;
+        constexpr bool kConst = !std::is_same_v<decltype(S_), int>;
+        constexpr int S = [] { if constexpr (kConst) return (int)decltype(S_)::value; else return 0; }();
+        const int rt = kConst ? 0 : (int)S_;
+        if constexpr (!kFuseA && u == 0) {
+            dma_b32<kOffS + S * (kSA + kSW)>(dSA, lds_s + rt * (kSA + kSW), sa_off0, s_fetch * sa_kstep);
+        } else if constexpr (u == kScaleDma - 1) {
+            dma_b32<kOffS + S * (kSA + kSW) + kSA>(dSW, lds_s + rt * (kSA + kSW), sw_off0,
+                                                   kRowW ? ((kb0 + s_fetch) >> 2) * sw_kstep : s_fetch * sw_kstep);
+        } else if constexpr (u < kScaleDma + kAUnits) {
+            constexpr int i = (u - kScaleDma) * (kPairA ? 2 : 1);
+            const int soff = s_fetch * (kFuseA ? 2 * kRowB : kRowB);
+            if constexpr (kPairA)
+                dma_b128_pair<S * kA + i * 1024, false>(dA, lds_a + rt * kA, a_off(i), a_off(i + 1), soff);
             else
-                dma_b32(dSW, base + kA + kB + kSA + wave * 256, live ? sw_off0 + s * sw_kstep : kOob);
-        } else if (d < kScaleDma + kAInstr) {
-            const int i = d - kScaleDma;
-            int off;
-            if constexpr (kFuseA) off = xa_off[i] + s * 2 * kRowB;
-            else if constexpr (kSorted) off = a_row[i] + ((i & 1) ? ch_o : ch_e) + k0;
-            else off = ((i & 1) ? a_o : a_e) + (int)(i * 8 * a.lda) + k0;
-            dma_b128(dA, base + (wave * kAInstr + i) * 1024, live && !((a_dead >> i) & 1u) ? off : kOob);
+                dma_b128<S * kA + i * 1024, false>(dA, lds_a + rt * kA, a_off(i), soff);
         } else {
-            const int i = d - kScaleDma - kAInstr;
-            const uint32_t dst = base + kA + (wave * kBInstr + i) * 1024;
-            const int off = live ? ((i & 1) ? w_o : w_e) + (int)(i * 8 * a.ldw) + k0 : kOob;
-            if constexpr (kWeightNt) dma_b128_nt(dW, dst, off);
-            else dma_b128(dW, dst, off);
+            constexpr int i = (u - kScaleDma - kAUnits) * (kPairW ? 2 : 1);
+            if constexpr (kPairW)
+                dma_b128_pair<kOffW + S * kB + i * 1024, kWeightNt>(dW, lds_w + rt * kB, w_off(i), w_off(i + 1),
+                                                                     s_fetch * kRowB);
+            else
+                dma_b128<kOffW + S * kB + i * 1024, kWeightNt>(dW, lds_w + rt * kB, w_off(i), s_fetch * kRowB);
         }
+    };
+    // Past the last block the descriptors end at 0, so the A and W loads write
+    // zeros and fetch nothing; every block issues the same loads, so the waits
+    // are constants and no load is branched around.
+    auto fetch_block = [&](int b) {
+        // all ones while b < KB; scalar instructions written out, as the
+        // compiler would turn the masks into vector selects
+        int more, na = dA[2], nw = dW[2];
+        asm("s_ashr_i32 %0, %1, 31" : "=s"(more) : "s"(b - KB) : "scc");
+        asm("s_and_b32 %0, %1, %2" : "=s"(s_fetch) : "s"(b), "s"(more) : "scc");
+        asm("s_and_b32 %0, %0, %1" : "+s"(na) : "s"(more) : "scc");
+        asm("s_and_b32 %0, %0, %1" : "+s"(nw) : "s"(more) : "scc");
+        dA[2] = na;
+        dW[2] = nw;
     };
 
     const int nb_local = (wn * TN) / 128;  // this wavefront's weight-scale block within the tile
@@ -593,31 +698,40 @@ gemm_bs_kernel(const GemmArgs a) {
     const int fs = (lane >> 1) & 7;
     const int frow = (lane & 31) * kRowB;
 
+#ifdef KBN_ACC_AGPR
+    constexpr bool kAccAgpr = kWaves == 4;
+#else
+    constexpr bool kAccAgpr = false;
+#endif
     v16f acc[FM][FN];
 #pragma unroll
     for (int i = 0; i < FM; ++i)
 #pragma unroll
         for (int j = 0; j < FN; ++j) acc[i][j] = v16f{};
 
-    auto stage_ptr = [&](int s) -> const uint8_t* { return smem + (s % kStages) * kStage; };
-    // 16-B read q (0 <= q < 2 (FM + FN)) of K half kk: half q % 2 of fragment
-    // q / 2, A fragments first
-    auto read_half = [&](const uint8_t* st, int kk, int q, v8i (&af)[FM], v8i (&bf)[FN]) {
-        const int f = q >> 1, h = q & 1;
-        const int c = 4 * kk + 2 * (lane >> 5) + h;
-        const uint8_t* tile = f < FM ? st + (wm * TM + f * 32) * kArow : st + kA + (wn * TN + (f - FM) * 32) * kRowB;
-        // fused A rows: tile row r at LDS row (r % 4) kAW + r / 4 (256 B each),
-        // chunk c in slot c ^ (r & 15); rows past 4 kAW (never stored) alias
-        // loaded ones so every read stays inside the stage's A rows
-        int off;
-        if (kFuseA && f < FM) {
-            const int r = wm * TM + f * 32 + (lane & 31);
-            off = ((r & 3) * kAW + ((r >> 2) & (kAW - 1))) * kArow + ((c ^ (r & 15)) << 4) -
-                  (int)(tile - st);
+    // per-lane LDS offsets of chunk j = 2 kk + h of the first A and W fragment
+    int a_rd[4], w_rd[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int c = 4 * (j >> 1) + 2 * (lane >> 5) + (j & 1);
+        if constexpr (kFuseA) {
+            // fused A rows: tile row r at LDS row (r % 4) kAW + r / 4 (256 B each), chunk c in slot
+            // c ^ (r & 15); rows past 4 kAW (never stored) alias loaded ones so every read stays
+            // inside the stage's A rows
+            static_assert(!kFuseA || FM == 1, "one A fragment per wavefront");
+            const int r = wm * TM + (lane & 31);
+            a_rd[j] = ((r & 3) * kAW + ((r >> 2) & (kAW - 1))) * kArow + ((c ^ (r & 15)) << 4);
         } else {
-            off = frow + ((c ^ fs) << 4);
+            a_rd[j] = wm * TM * kRowB + frow + ((c ^ fs) << 4);
         }
-        const v4i v = *reinterpret_cast<const v4i*>(tile + off);
+        w_rd[j] = wn * TN * kRowB + frow + ((c ^ fs) << 4);
+    }
+    // 16-B read q (0 <= q < 2 (FM + FN)) of K half kk of stage S: half q % 2
+    // of fragment q / 2, A fragments first
+    auto read_half = [&](int S, int kk, int q, v8i (&af)[FM], v8i (&bf)[FN]) {
+        const int f = q >> 1, h = q & 1, j = 2 * kk + h;
+        const v4i v = f < FM ? *reinterpret_cast<const v4i*>(smem + a_rd[j] + (S * kA + f * 32 * kArow))
+                             : *reinterpret_cast<const v4i*>(smem + w_rd[j] + (kOffW + S * kB + (f - FM) * 32 * kRowB));
         if (f < FM) {
             if (h) af[f].hi = v; else af[f].lo = v;
         } else {
@@ -629,22 +743,23 @@ gemm_bs_kernel(const GemmArgs a) {
     // kRowW: the packed word of each fragment's W row (lane & 31)
     // kFragW: the fp32 block scale (as bits) of each fragment's 32 W rows
     uint32_t swr[kPerFragW ? FN : 1], nswr[kPerFragW ? FN : 1];
-    auto read_scales = [&](const uint8_t* st, float (&sa)[FM], float& sw, uint32_t (&wr)[kPerFragW ? FN : 1]) {
-        const float* ssa = reinterpret_cast<const float*>(st + kA + kB);
+    auto read_scales = [&](int S, float (&sa)[FM], float& sw, uint32_t (&wr)[kPerFragW ? FN : 1]) {
+        const uint8_t* sc = smem + kOffS + S * (kSA + kSW);
+        const float* ssa = reinterpret_cast<const float*>(sc);
 #pragma unroll
         for (int i = 0; i < FM; ++i) sa[i] = ssa[wm * TM + i * 32 + (lane & 31)];
         if constexpr (kRowW) {
-            const uint32_t* sww = reinterpret_cast<const uint32_t*>(st + kA + kB + kSA);
+            const uint32_t* sww = reinterpret_cast<const uint32_t*>(sc + kSA);
 #pragma unroll
             for (int j = 0; j < FN; ++j) wr[j] = sww[wn * TN + j * 32 + (lane & 31)];
             sw = 0.f;
         } else if constexpr (kFragW) {
-            const uint32_t* ssw = reinterpret_cast<const uint32_t*>(st + kA + kB + kSA + wave * 256);
+            const uint32_t* ssw = reinterpret_cast<const uint32_t*>(sc + kSA + wave * 256);
 #pragma unroll
             for (int j = 0; j < FN; ++j) wr[j] = ssw[((n0 & 127) + wn * TN + j * 32) >> 7];
             sw = 0.f;
         } else {
-            const float* ssw = reinterpret_cast<const float*>(st + kA + kB + kSA + wave * 256);
+            const float* ssw = reinterpret_cast<const float*>(sc + kSA + wave * 256);
             sw = ssw[nb_local];
         }
     };
@@ -660,7 +775,7 @@ gemm_bs_kernel(const GemmArgs a) {
             for (int j = 0; j < FN; ++j) e[j] = (int)((wr[j] >> (8 * (gkb & 3))) & 0xFFu);
         } else if constexpr (kFragW) {
 #pragma unroll
-            for (int j = 0; j < FN; ++j) e[j] = ue8m0_ceil_byte(__uint_as_float(wr[j]));
+            for (int j = 0; j < FN; ++j) e[j] = ue8m0_ceil_top(__uint_as_float(wr[j]));
             (void)gkb;
         }
     };
@@ -680,26 +795,26 @@ gemm_bs_kernel(const GemmArgs a) {
             row_live[i] = r < a.M && a.expert_ids[r] == expert;
         }
     }
-    // E8M0 bytes of raw scales; FP32 contract: the first block's mantissa
+    // E8M0 operands of raw scales (in the top byte); FP32 contract: the first block's mantissa
     // products (step < 0), or the ratios to the next block's products, which
     // then become current (their block follows)
     auto convert = [&](const float (&s)[FM], float w, int (&e)[FM], int& f, int step) {
         if constexpr (kUe8m0) {
 #pragma unroll
-            for (int i = 0; i < FM; ++i) e[i] = ue8m0_ceil_byte(s[i]);
-            f = ue8m0_ceil_byte(w);
+            for (int i = 0; i < FM; ++i) e[i] = ue8m0_ceil_top(s[i]);
+            f = ue8m0_ceil_top(w);
         } else {
             const float mw = scale_mant(w);
             float m[FM];
             bool diff = false;
 #pragma unroll
             for (int i = 0; i < FM; ++i) {
-                e[i] = scale_exp_byte(s[i]);
+                e[i] = scale_exp_top(s[i]);
                 m[i] = scale_mant(s[i]) * mw;
                 if constexpr (kGrouped) m[i] = row_live[i] ? m[i] : 1.f;
                 diff |= m[i] != mu[i];
             }
-            f = scale_exp_byte(w);
+            f = scale_exp_top(w);
             if (step >= 0) {
                 // the quotient of two different values in [1, 4) is never 1,
                 // so the divisions are needed exactly when a product changed
@@ -721,8 +836,9 @@ gemm_bs_kernel(const GemmArgs a) {
     // block's scales enter as E8M0 operands: eb for the W rows, ea[i] per A row.
     auto mfma_at = [&](int t, const v8i (&fa)[FM], const v8i (&fb)[FN]) {
         const int i = t / FN, j = t % FN;
-        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[j], fa[i], acc[i][j], 0, 0, 0,
-                                                                      kPerFragW ? ebr[j] : eb, 0, ea[i]);
+        acc[i][j] = __builtin_amdgcn_mfma_scale_f32_32x32x64_f8f6f4(fb[j], fa[i], acc[i][j], 0, 0, kRowW ? 0 : 3,
+                                                                      kPerFragW ? ebr[j] : eb, 3, ea[i]);
+        keep_here<kAccAgpr>(acc[i][j][0]);
     };
     // FP32 contract: bring the running sum to the new block's mantissa base
     // before the block's first MFMA.  One uniform branch around all of it,
@@ -733,9 +849,7 @@ gemm_bs_kernel(const GemmArgs a) {
 #pragma unroll
                 for (int i = 0; i < FM; ++i)
 #pragma unroll
-                    for (int j = 0; j < FN; ++j)
-#pragma unroll
-                        for (int r = 0; r < 16; ++r) acc[i][j][r] = acc[i][j][r] * ratio[i];
+                    for (int j = 0; j < FN; ++j) acc[i][j] *= ratio[i];
             }
         }
     };
@@ -758,12 +872,12 @@ gemm_bs_kernel(const GemmArgs a) {
     // scale the stage's activation-scale slot.  Every lane's loads complete
     // before the first write (the DPP max consumes them all), and no other
     // wavefront reads these rows before the next barrier.
-    auto quant_rows = [&](const uint8_t* st_c) {
+    auto quant_rows = [&](int S) {
         if constexpr (kFuseA) {
             typedef uint16_t u16v2 __attribute__((ext_vector_type(2)));
             constexpr int kQ = kFuseA;            // 16-B bf16 chunks per lane
             constexpr int kLanes = 16 / kQ;       // lanes per row
-            uint8_t* st = const_cast<uint8_t*>(st_c);
+            uint8_t* st = smem + S * kA;
             const int pl = lane / kLanes;         // row of this wave: LDS row 16 w + pl
             const int r = wave + 4 * pl, sr = r & 15;
             const int c0 = (lane % kLanes) * kQ;  // first bf16 chunk of the lane
@@ -835,9 +949,9 @@ gemm_bs_kernel(const GemmArgs a) {
                     *reinterpret_cast<u32x4*>(row + ((((c0 + q) >> 1) ^ sr) << 4)) =
                         u32x4{c[2 * q], c[2 * q + 1], c[2 * q + 2], c[2 * q + 3]};
             }
-            if (lane % kLanes == 0) reinterpret_cast<float*>(st + kA + kB)[r] = sc;
+            if (lane % kLanes == 0) reinterpret_cast<float*>(smem + kOffS + S * (kSA + kSW))[r] = sc;
         } else {
-            (void)st_c;
+            (void)S;
         }
     };
 
@@ -860,23 +974,32 @@ gemm_bs_kernel(const GemmArgs a) {
     }
     auto want = [&](int q) { return !kGrouped || ((q >> 1) < FM ? (q >> 1) < nlive : nlive > 0); };
     // prologue: blocks 0 .. kStages-1 in flight, block 0 published
-#pragma unroll
-    for (int s = 0; s < kStages; ++s)
-#pragma unroll
-        for (int d = 0; d < kDma; ++d) issue_one(s, s < KB, d);
+    static_for<kStages>([&](auto S_) {
+        fetch_block(decltype(S_)::value);
+        static_for<kUnits>([&](auto u_) { issue_unit(S_, u_); });
+    });
     wait_dma_n<(kStages - 1) * kDma>();
-    quant_rows(stage_ptr(0));   // fused A: block 0 (the loop quantizes block kb+1 in iteration kb)
+    quant_rows(0);   // fused A: block 0 (the loop quantizes block kb+1 in iteration kb)
     __syncthreads();
-    read_scales(stage_ptr(0), sa, sw, swr);
+    read_scales(0, sa, sw, swr);
 #pragma unroll
     for (int q = 0; q < kR; ++q)
-        if (want(q)) read_half(stage_ptr(0), 0, q, fa0, fb0);
+        if (want(q)) read_half(0, 0, q, fa0, fb0);
 
     convert(sa, sw, ea, eb, -1);
     row_bytes(swr, kb0, ebr);
 
-    for (int kb = 0; kb < KB; ++kb) {
-        const uint8_t* cur = stage_ptr(kb);
+    // K block kb, in stage S.  kFetch: block kb+kStages is fetched into S;
+    // otherwise kb is one of the last KB % kStages blocks, which have nothing
+    // left to fetch.
+    auto block = [&](auto S_, auto fetch_, int kb) {
+        constexpr bool kFetch = decltype(fetch_)::value;
+        const int S = S_, next = S + 1 < kStages ? S + 1 : 0;
+        // blocks' loads issued after those of block kb+1
+        constexpr int kAhead = [] {
+            if constexpr (kFetch) return kStages - 2;
+            else return std::max(kStages - 2 - (int)decltype(S_)::value, 0);
+        }();
         rescale_all();
         // ---- sub-step 0: K half 0 of block kb; read K half 1
 #pragma unroll
@@ -884,7 +1007,7 @@ gemm_bs_kernel(const GemmArgs a) {
             if (!kGrouped || t / FN < nlive) mfma_at(t, fa0, fb0);
 #pragma unroll
             for (int q = t * kR / kT; q < (t + 1) * kR / kT; ++q)
-                if (want(q)) read_half(cur, 1, q, fa1, fb1);
+                if (want(q)) read_half(S, 1, q, fa1, fb1);
             __builtin_amdgcn_sched_barrier(0);
         }
 
@@ -893,40 +1016,42 @@ gemm_bs_kernel(const GemmArgs a) {
         // from L2 ahead of the block's weights, which may still stream in);
         // the hand-off below publishes the codes with the weights
         if constexpr (kFuseA) {
-            wait_dma_n<(kStages - 2) * kDma + kBInstr>();
-            quant_rows(stage_ptr(kb + 1));
+            wait_dma_n<kAhead * kDma + kBInstr>();
+            quant_rows(next);
         }
 
-        // ---- hand-off: publish block kb+1, free buffer kb for block kb+kStages
-        wait_dma_n<(kStages - 2) * kDma>();
+        // ---- hand-off: publish block kb+1, free stage S for block kb+kStages
+        wait_dma_n<kAhead * kDma>();
         wait_lds();
         __syncthreads();
+        if constexpr (kFetch) fetch_block(kb + kStages);
 
         // ---- sub-step 1: K half 1 of block kb; read K half 0 of block kb+1
-        // (past the last block this reads a zero-filled buffer, unused) and
-        // DMA block kb+kStages into the freed buffer
-        const uint8_t* nxt = stage_ptr(kb + 1);
-        const int snext = kb + kStages;
-        const bool live = snext < KB;
-#pragma unroll
-        for (int t = 0; t < kT; ++t) {
+        // (past the last block this reads a zero-filled stage, unused) and DMA
+        // block kb+kStages into the freed stage
+        static_for<kT>([&](auto t_) {
+            constexpr int t = decltype(t_)::value;
             if (!kGrouped || t / FN < nlive) mfma_at(t, fa1, fb1);
-            if (t == 0) read_scales(nxt, nsa, nsw, nswr);
+            if constexpr (t == 0) read_scales(next, nsa, nsw, nswr);
             // converted scales of block kb+1, half a sub-step after their
             // reads (FP32 contract: none past the last block, whose mantissa
             // products the store needs)
-            if (t == kT / 2) {
+            if constexpr (t == kT / 2) {
                 if constexpr (kUe8m0) convert(nsa, nsw, nea, neb, kb);
                 else if (kb + 1 < KB) convert(nsa, nsw, nea, neb, kb);
                 row_bytes(nswr, kb0 + kb + 1, nebr);
             }
 #pragma unroll
             for (int q = t * kR / kT; q < (t + 1) * kR / kT; ++q)
-                if (want(q)) read_half(nxt, 0, q, fa0, fb0);
-#pragma unroll
-            for (int d = t * kDma / kT; d < (t + 1) * kDma / kT; ++d) issue_one(snext, live, d);
+                if (want(q)) read_half(next, 0, q, fa0, fb0);
+            if constexpr (kFetch) {
+                constexpr int u0 = t * kUnits / kT, u1 = (t + 1) * kUnits / kT;
+                static_for<u1 - u0>([&](auto u_) {
+                    issue_unit(S_, std::integral_constant<int, u0 + decltype(u_)::value>{});
+                });
+            }
             __builtin_amdgcn_sched_barrier(0);
-        }
+        });
         // FP32 contract: the running sum is kept in units of the current
         // block's mantissa product, S_kb = S_{kb-1} mu_{kb-1} / mu_kb + 2^e P_kb
         // (rescale_at applies the ratio as block kb+1 starts), so the true
@@ -939,6 +1064,27 @@ gemm_bs_kernel(const GemmArgs a) {
 #pragma unroll
             for (int j = 0; j < FN; ++j) ebr[j] = nebr[j];
         }
+    };
+    // With one wavefront per SIMD an instruction issues about every four
+    // cycles, so on the smaller tiles the loop is bound by how many there
+    // are, not by the 64-cycle MFMAs.  The stages are therefore unrolled:
+    // every LDS address is a register plus an instruction offset, the M0 of a
+    // load a register plus a literal, the K position one scalar (about 60
+    // instructions a block for a 128x64 tile's wavefront, 120 with the stage
+    // computed).  us a call, stage computed -> unrolled: 8 x 10240 x 8192
+    // 19.0 -> 17.4, 64 x 2048 x 2048 9.3 -> 8.9, 4096 x 36864 x 7168 836 ->
+    // 805.  The 128x256 MoE tiles stay as they were: in the larger loop the
+    // compiler moved their accumulators between register files (the experts
+    // layer 12% slower at 4096 tokens).
+    if constexpr (!((kGrouped || kSorted) && FM * FN >= 8)) {
+        int kb = 0;
+        for (; kb + kStages <= KB; kb += kStages)
+            static_for<kStages>([&](auto S_) { block(S_, std::true_type{}, kb + decltype(S_)::value); });
+        static_for<kStages - 1>([&](auto S_) {
+            if (kb + decltype(S_)::value < KB) block(S_, std::false_type{}, kb + decltype(S_)::value);
+        });
+    } else {
+        for (int kb = 0, st = 0; kb < KB; ++kb, st = st + 1 < kStages ? st + 1 : 0) block(st, std::true_type{}, kb);
     }
     // the trailing (out-of-range) loads still target this workgroup's LDS
     wait_dma();
@@ -950,9 +1096,7 @@ gemm_bs_kernel(const GemmArgs a) {
 #pragma unroll
             for (int i = 0; i < FM; ++i)
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = acc[i][j][r] * mu[i];
+                for (int j = 0; j < FN; ++j) acc[i][j] *= mu[i];
         }
     }
 
@@ -1042,9 +1186,7 @@ gemm_bs_kernel(const GemmArgs a) {
             if (a.row_weight) {
                 const float f = out_row[i] >= 0 ? a.row_weight[out_row[i]] : 0.f;
 #pragma unroll
-                for (int j = 0; j < FN; ++j)
-#pragma unroll
-                    for (int r = 0; r < 16; ++r) acc[i][j][r] = acc[i][j][r] * f;
+                for (int j = 0; j < FN; ++j) acc[i][j] *= f;
             }
         }
     }

@@ -85,15 +85,6 @@ __device__ __forceinline__ float ue8m0_ceil_div448(float amax) {
     return __uint_as_float((e - 8u + ((u & 0x7FFFFFu) > 0x600000u ? 1u : 0u)) << 23);
 }
 
-// Biased exponent byte (E8M0) of ue8m0_ceil(r): the per-operand scale
-// consumed by the block-scaled MFMA.
-__device__ __forceinline__ int ue8m0_ceil_byte(float r) {
-    uint32_t u = __float_as_uint(r);
-    uint32_t e = (u >> 23) & 0xFFu;
-    if (u & 0x7FFFFFu) e += 1;
-    return (int)(e > 254u ? 254u : e);
-}
-
 // Exact reciprocal of a power of two in the normal range.
 __device__ __forceinline__ float pow2_recip(float s) {
     uint32_t e = (__float_as_uint(s) >> 23) & 0xFFu;

@@ -46,6 +46,23 @@ def test_gemm_matches_oracle(gpu_device, M, N, K, ue8m0):
     assert_gemm_close(D, ref, f"gemm {M}x{N}x{K} ue8m0={ue8m0}")
 
 
+@pytest.mark.parametrize("ue8m0", [True, False])
+@pytest.mark.parametrize("M", [20, 100, 300])
+def test_gemm_k_blocks_against_stages(gpu_device, M, ue8m0):
+    """Every number of K blocks from one to nine, i.e. fewer than a tile's LDS
+    stages (two to four), whole rounds of them and every remainder, on 64-,
+    128- and 256-row tiles; 23 blocks may be split over K."""
+    N = 320
+    for KB in (1, 2, 3, 4, 5, 6, 7, 8, 9, 23):
+        K = 128 * KB
+        qa, sa, qw, sw = quantized_gemm_inputs(M, N, K, seed=M + KB)
+        if not ue8m0:
+            sw = (sw * np.float32(1.37)).astype(np.float32)
+        ref = oracle.gemm_nt_sample(qa, sa, qw, sw, ue8m0=ue8m0)
+        D = _gemm_gpu(qa, sa, qw, sw, gpu_device, ue8m0=ue8m0, col_major=KB % 2 == 0)
+        assert_gemm_close(D, ref, f"gemm {M}x{N}, {KB} K blocks, ue8m0={ue8m0}")
+
+
 def test_gemm_row_major_scales_and_ragged_n(gpu_device):
     M, N, K = 77, 200, 512
     qa, sa, qw, sw = quantized_gemm_inputs(M, N, K, seed=9)
