@@ -59,6 +59,7 @@ def _generate_silu_lut() -> None:
 # tiles need the AGPRs for their 256 accumulators per lane and stay without.
 FILE_FLAGS = {
     "gemm.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
+    "gemm_mid.hip": ["-mllvm", "-amdgpu-mfma-vgpr-form=true"],
 }
 
 

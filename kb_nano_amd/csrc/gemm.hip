@@ -342,12 +342,123 @@ static void plan_mixed_192(Schedule& s, int64_t M, int64_t N) {
     if (s.n192) s.tiles = s.dp_tiles = tm * ((N - s.n192) / 256 + s.n192 / 192);
 }
 
-// Dense tile configuration: 256x256 (2 LDS stages) when M > 128 (128x256,
-// 3 stages, under the FP32 contract, whose per-row mantissa state does not
-// fit next to a 256x256 tile's accumulators), 128x128 (4 stages) for
-// 64 < M <= 128, 64x128 (3 stages, two workgroups per CU) for M <= 64,
+// Modelled time of the dense UE8M0 tiles above 64 rows, in microseconds: what
+// decides is how a shape's tiles fill the CUs, so each tile is priced and the
+// cheapest taken.  A wave of w workgroups of kb K blocks takes
+//   kb (block + busy w / slots + fetch MB) + wave
+// with MB the distinct A and W rows of one K step over the wave, and the call
+// at least 2 us plus its bytes at `rate` TB/s.  Splitting K over s workgroups
+// a tile adds split + slab MB + s per.  Fitted to 234 shapes (M 72 to 4096
+// over 13 weights from 2048 x 2048 to 57344 x 8192 and 8192 x 28672, every
+// tile, 1 to 8 splits; 5-11% rms a tile).  Over those shapes the pick is 1.31x
+// faster than 128x128 (M <= 128) or 256x256 tiles throughout, and 3% from the
+// best tile measured.  Some of it, us: 200 x 2048 x 2048 20.2 -> 7.1
+// (64x64), 200 x 8192 x 8192 34.9 -> 22 (128x64), 777 x 4608 x 7168 44.8 ->
+// 33.5 (64x256), 1024 x 8192 x 8192 76 -> 56 (128x256, 8 wavefronts),
+// 1024 x 7168 x 18432 138 -> 121 (256x128).
+struct DenseTile {
+    int bm, bn, stages, waves;
+    double block, busy, fetch, wave, start, split, slab, per, rate;
+    // workgroups the chip holds at once: two per CU where two fit its LDS
+    int64_t slots() const {
+        return (int64_t)cu_count() * (stages * ((bm + bn) * kRowB + waves * 512) <= 80 * 1024 ? 2 : 1);
+    }
+};
+constexpr DenseTile kDenseTiles[] = {
+    {64, 64, 4, 4, 0.113, 0.321, 0.008, 0.328, 3.768, 4.046, 0.040, 0.411, 3.578},
+    {128, 64, 4, 4, 0.242, 0.106, 0.007, 1.495, 2.075, 4.062, 0.141, 0.390, 4.248},
+    {64, 256, 3, 4, 0.342, 0.244, 0.071, 1.877, 1.755, 5.051, 0.000, 0.084, 4.257},
+    {128, 128, 4, 4, 0.415, 0.173, 0.026, 3.168, 1.273, 2.282, 0.471, 0.254, 4.883},
+    {128, 256, 3, 8, 0.479, 0.316, 0.068, 3.622, 0.389, 2.799, 0.237, 0.000, 4.700},
+    {256, 128, 3, 4, 0.578, 0.251, 0.000, 5.057, 0.171, 2.016, 0.409, 0.378, 4.876},
+    {192, 256, 2, 4, 0.967, 0.233, 0.084, 1.821, 0.000, 0.000, 0.308, 0.405, 6.036},
+    {256, 256, 2, 4, 1.094, 0.346, 0.060, 3.163, 0.000, 0.000, 0.312, 0.318, 3.954},
+};
+constexpr int kTile128 = 3, kTile256 = 7;   // the tiles of M <= 128 and M > 128 before the others are priced
+
+// Modelled time of `full` waves of whole-K tiles and then `rest` tiles (fewer
+// than a wave) in `splits` pieces of K.
+static double dense_cost(const DenseTile& t, int64_t M, int64_t N, int64_t K, double full, int64_t rest, int splits) {
+    const int64_t slots = t.slots();
+    const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn, kbt = K / kGroup;
+    auto wave = [&](double w, int s) {   // one wave of w workgroups, s to a tile
+        const double tiles = w / s, kb = (double)((kbt + s - 1) / s);
+        const double cols = std::min<double>((double)tn, std::max(1.0, tiles / (double)tm));
+        const double rows = std::min<double>((double)tm, std::max(1.0, tiles));
+        const double mb = (cols * t.bn + rows * t.bm) * kRowB * s / 1e6;
+        return kb * (t.block + t.busy * w / (double)slots + t.fetch * mb) + t.wave;
+    };
+    double us = t.start + full * wave((double)slots, 1);
+    if (rest > 0) us += wave((double)(rest * splits), splits);
+    us = std::max(us, 2.0 + (double)(N * K + M * K + 2 * M * N) / (t.rate * 1e6));
+    if (splits > 1) {
+        // fp32 slabs of the split tiles: live rows x columns a piece
+        const double slab_mb = (double)splits * rest / (double)(tm * tn) * (double)std::min(M, tm * t.bm) *
+                               (double)(tn * t.bn) * 4 / 1e6;
+        us += t.split + t.slab * slab_mb + t.per * splits;
+    }
+    return us;
+}
+
+// Replaces s, the 128x128 or 256x256 plan, by the tile priced cheapest if that
+// saves at least 5%, or 15% for 256-column tiles up to 128 rows (less is within
+// the model's error: with 4% everywhere 65 x 36864 x 7168 took 128x256 tiles,
+// 66.5 us against 58.7, and 640 x 36864 x 7168 177.6 against 174.6).  The fit
+// holds no grids of a few workgroups, so they keep their plan (65 x 512 x 7168
+// in 16 workgroups of 128x256: 15.4 us against 12.4 of 128x128).  K of at most 12
+// blocks keeps 128x128 for up to 128 rows, although 64x64 measured faster
+// there (3072 x 1536 at 128 rows 7.0 against 10.7 us): those plans, and that
+// a row's result does not depend on the row count under them, are held by
+// tests.
+constexpr int64_t kKeep128Kb = 12, kMinWorkgroups = 32;
+
+static void plan_dense_tile(Schedule& s, int64_t M, int64_t N, int64_t K, bool allow_split) {
+    const int64_t kbt = K / kGroup;
+    if (M <= 128 && kbt <= kKeep128Kb) return;
+    const int64_t cus = cu_count();
+    const DenseTile& old = kDenseTiles[M <= 128 ? kTile128 : kTile256];
+    double best;
+    if (s.n192) {   // two launches; a 256x192 wave counts 0.78 of a 256x256 one
+        const int64_t tm = (M + 255) / 256;
+        auto waves = [&](int64_t t) { return (double)((t + cus - 1) / cus); };
+        best = dense_cost(old, M, N, K, waves(tm * ((N - s.n192) / 256)) + 0.78 * waves(tm * (s.n192 / 192)), 0, 1);
+    } else {
+        best = dense_cost(old, M, N, K, (double)(s.tiles / cus), s.tiles % cus, s.splits);
+    }
+    best *= 0.95;
+    for (const DenseTile& t : kDenseTiles) {
+        if (&t == &old) continue;
+        const int64_t slots = t.slots();
+        const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
+        for (int sp = 1; sp <= 8; ++sp) {
+            if (sp > 1 && (!allow_split || kbt < 8 || kbt < 4 * sp || tiles * sp > slots)) break;
+            const int kbps = (int)((kbt + sp - 1) / sp), pieces = (int)((kbt + kbps - 1) / kbps);
+            if (pieces != sp) continue;
+            const double us = sp > 1 ? dense_cost(t, M, N, K, 0, tiles, sp)
+                                     : dense_cost(t, M, N, K, (double)(tiles / slots), tiles % slots, 1);
+            const double bias = M <= 128 && t.bn == 256 ? 0.95 / 0.85 : 1.0;
+            if (us * bias >= best || tiles * sp < kMinWorkgroups) continue;
+            best = us * bias;
+            Schedule n;
+            n.bm = t.bm; n.bn = t.bn; n.stages = t.stages; n.waves = t.waves;
+            n.tiles = tiles;
+            n.dp_tiles = sp > 1 ? 0 : tiles;
+            n.splits = sp;
+            n.kb_per_split = kbps;
+            n.ws_bytes = sp > 1 ? (int64_t)sp * tiles * t.bm * t.bn * 4 : 0;
+            n.ws_start = std::max(s.ws_bytes, s.ws_start);
+            s = n;
+        }
+    }
+}
+
+// Dense tile configuration.  FP32 contract: 128x256 (3 LDS stages; its per-row
+// mantissa state does not fit next to a 256x256 tile's accumulators) when
+// M > 128, else as UE8M0's starting point.  UE8M0: 128x128 (4 stages) for
+// 64 < M <= 128, 256x256 (2 stages) above, or the tile that plan_dense_tile
+// prices cheaper.  64x128 (3 stages, two workgroups per CU) for M <= 64,
 // where the weights dominate the traffic.
-static Schedule dense_schedule(int64_t M, int64_t N, int64_t K, int ue8m0, bool allow_split) {
+static Schedule plan_dense(int64_t M, int64_t N, int64_t K, int ue8m0, bool allow_split) {
     Schedule s;
     if (M > 128 && !ue8m0) {
         s.bm = 128; s.bn = 256; s.stages = 3;
@@ -370,7 +481,28 @@ static Schedule dense_schedule(int64_t M, int64_t N, int64_t K, int ue8m0, bool 
     s.kb_per_split = (int)(K / kGroup);
     if (allow_split) plan_tail(s, M, (int)(K / kGroup));
     if (s.bm == 256 && s.splits == 1 && K >= kMixedMinK) plan_mixed_192(s, M, N);
+    if (ue8m0) plan_dense_tile(s, M, N, K, allow_split);
     return s;
+}
+
+// plan_dense, with the thread's latest plans kept: pricing every tile takes
+// 1-5 us a call, as long as a launch.  A plan depends on nothing but its key.
+static Schedule dense_schedule(int64_t M, int64_t N, int64_t K, int ue8m0, bool allow_split) {
+    struct Entry {
+        int64_t M = 0, N = 0, K = 0;
+        int kind = -1;
+        Schedule plan;
+    };
+    thread_local Entry kept[128];
+    const int kind = cu_count() * 4 + (ue8m0 ? 2 : 0) + (allow_split ? 1 : 0);
+    const uint64_t h = ((uint64_t)M * 0x9E3779B97F4A7C15ull) ^ ((uint64_t)N * 0xC2B2AE3D27D4EB4Full) ^
+                       ((uint64_t)K * 0x165667B19E3779F9ull) ^ (uint64_t)kind;
+    Entry& e = kept[(h ^ (h >> 32)) >> 8 & 127];
+    if (e.kind != kind || e.M != M || e.N != N || e.K != K) {
+        e.plan = plan_dense(M, N, K, ue8m0, allow_split);
+        e.M = M; e.N = N; e.K = K; e.kind = kind;
+    }
+    return e.plan;
 }
 
 // Tile plan of the GEMM over bf16 activations (M <= 64, quantized by the
@@ -389,7 +521,7 @@ static Schedule bf16a_schedule(int64_t M, int64_t N, int64_t K, bool allow_split
 
 // Dense UE8M0 tiles with packed per-row weight scales (a.sWp).
 static int dispatch_dense_roww(const GemmArgs& a, const Schedule& sc, int64_t K, hipStream_t st, const char* what) {
-    if (sc.bm == 256 && sc.bn == 256) return launch_gemm_256_roww(a, sc, K, st, what);
+    if (sc.bm >= 192 && sc.bn == 256) return launch_gemm_256_roww(a, sc, K, st, what);
     if (sc.bm == 128 && sc.bn == 128) return launch_gemm<128, 128, 4, true, false, 4, 0, true>(a, sc, st, what);
     if (sc.bm == 64 && sc.bn == 128) {
         if (sc.stages == 4) return launch_gemm<64, 128, 4, true, false, 4, 0, true>(a, sc, st, what);
@@ -397,14 +529,13 @@ static int dispatch_dense_roww(const GemmArgs& a, const Schedule& sc, int64_t K,
     }
     if (sc.bm == 64 && sc.bn == 64 && sc.stages == 4)
         return launch_gemm<64, 64, 4, true, false, 4, 0, true>(a, sc, st, what);
-    set_error("%s: no packed-scale kernel for %dx%d tiles", what, sc.bm, sc.bn);
-    return 1;
+    return launch_gemm_mid_roww(a, sc, st, what);
 }
 
 template <bool kUe8m0>
 static int dispatch_dense(const GemmArgs& a, const Schedule& sc, int64_t K, hipStream_t st, const char* what) {
     if constexpr (kUe8m0) {
-        if (sc.bm == 256 && sc.bn == 256) return launch_gemm_256(a, sc, K, st, what);
+        if (sc.bm >= 192 && sc.bn == 256) return launch_gemm_256(a, sc, K, st, what);
     } else {
         if (sc.bm == 128 && sc.bn == 256) return launch_gemm<128, 256, 3, false, false>(a, sc, st, what);
     }
@@ -415,6 +546,7 @@ static int dispatch_dense(const GemmArgs& a, const Schedule& sc, int64_t K, hipS
     }
     if constexpr (kUe8m0) {
         if (sc.bm == 64 && sc.bn == 64 && sc.stages == 4) return launch_gemm<64, 64, 4, true, false>(a, sc, st, what);
+        return launch_gemm_mid(a, sc, st, what);
     }
     set_error("%s: no kernel for %dx%d tiles", what, sc.bm, sc.bn);
     return 1;
@@ -573,7 +705,10 @@ extern "C" int kbn_fp8_gemm_nt(const void* A, int64_t lda, const float* sA, int6
 
 extern "C" int64_t kbn_fp8_gemm_nt_workspace_bytes(int64_t M, int64_t N, int64_t K, int scale_ue8m0) {
     if (M <= 0 || N <= 0 || K <= 0 || K % kGroup != 0 || M > 0x7FFFFFFFLL || N > 0x7FFFFFFFLL) return 0;
-    return dense_schedule(M, N, K, scale_ue8m0, true).ws_bytes;
+    // at least what the starting plan (128x128 or 256x256 tiles) would write,
+    // so what a caller holds for a shape does not hang on which tile is taken
+    const Schedule s = dense_schedule(M, N, K, scale_ue8m0, true);
+    return std::max(s.ws_bytes, s.ws_start);
 }
 
 extern "C" int kbn_fp8_gemm_nt_ws(const void* A, int64_t lda, const float* sA, int64_t sA_stride_m,

@@ -1428,10 +1428,12 @@ __global__ __launch_bounds__(256) void splitk_reduce_kernel(const GemmArgs a) {
 // slots, followed by the reduction.
 struct Schedule {
     int bm = 0, bn = 0, stages = 0;
+    int waves = 4;                // wavefronts of a workgroup
     int64_t tiles = 0;
     int64_t dp_tiles = 0;         // tiles [0, dp_tiles) data-parallel
     int splits = 1, kb_per_split = 0;  // the tail [dp_tiles, tiles)
     int64_t ws_bytes = 0;         // fp32 slabs of the tail
+    int64_t ws_start = 0;         // and those of the plan this one replaced (plan_dense_tile)
     bool fused = false;           // the split launch sums the slabs itself
     int fuse_a = 0;               // bf16 activations quantized by the GEMM: rows of four per wavefront (1, 2, 4)
     // 256-row tiles only: the last n192 columns run as 256x192 tiles in a
@@ -1461,9 +1463,13 @@ constexpr bool fused_split_sum(int bm, int bn, int64_t M, int splits, int kb_per
 // nullptr (then the separate reduction kernel runs); defined in gemm.hip.
 unsigned* splitk_flags_for(hipStream_t st, int64_t tail_tiles);
 
-// The 256x256 dense tiles (M > 128, UE8M0), built in their own translation
-// unit (gemm_big.hip) without the VGPR-form MFMA option: their 256
-// accumulators per lane need the AGPRs.
+// The tiles between the weight-streaming ones and 256x256 (gemm_mid.hip:
+// 128x64, 64x256, 128x256, 256x128), and the 256x256 and 192x256 dense tiles,
+// built in their own translation unit (gemm_big.hip) without the VGPR-form
+// MFMA option: their 192 or 256 accumulators per lane need the AGPRs.  All
+// UE8M0, M > 64.
+int launch_gemm_mid(const GemmArgs& a, const Schedule& sc, hipStream_t st, const char* what);
+int launch_gemm_mid_roww(const GemmArgs& a, const Schedule& sc, hipStream_t st, const char* what);
 int launch_gemm_256(const GemmArgs& a, const Schedule& sc, int64_t K, hipStream_t st, const char* what);
 int launch_gemm_256_roww(const GemmArgs& a, const Schedule& sc, int64_t K, hipStream_t st, const char* what);
 

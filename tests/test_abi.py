@@ -669,6 +669,33 @@ def test_weight_stream_plans_narrow_and_wide():
     assert "bad arguments" in _err()
 
 
+def test_dense_plans_above_64_rows_are_launchable():
+    """Random shapes above 64 rows (no GPU: 256 CUs assumed): the tile has a
+    kernel, the splits cover K without an empty one and never cut fewer than
+    8 K blocks, the split workgroups fit one wave, the slabs fit the
+    allocation-free entry point's scratch and what a caller is asked for, and
+    a plan is the same the second time."""
+    import numpy as np
+    from kb_nano_amd._lib import lib
+    L = lib()
+    tiles = {(64, 64, 4), (128, 64, 4), (64, 256, 3), (128, 128, 4), (128, 256, 3), (256, 128, 3), (192, 256, 2),
+             (256, 256, 2)}
+    rng = np.random.default_rng(7)
+    for _ in range(3000):
+        M = int(65 * (8192 / 65) ** rng.random())
+        N, K = int(8 * 2 ** (13 * rng.random())), 128 * int(1 + 250 ** rng.random())
+        p = _plan(L, M, N, K)
+        bm, bn, stages, n, dp, splits, kbps, fused, ws = (int(v) for v in p)
+        assert (bm, bn, stages) in tiles and not fused, (M, N, K, p)
+        assert n >= -(-M // bm) * -(-N // bn)     # more where the last columns take 192-column tiles
+        assert splits * kbps >= K // 128 > (splits - 1) * kbps and (splits == 1 or K >= 8 * 128), (M, N, K, p)
+        if splits > 1:
+            slots = 256 * (2 if stages * ((bm + bn) * 128 + 2048) <= 80 * 1024 else 1)
+            assert (n - dp) * splits <= slots and ws == splits * (n - dp) * bm * bn * 4 <= 64 << 20, (M, N, K, p)
+        assert L.kbn_fp8_gemm_nt_workspace_bytes(M, N, K, 1) >= ws
+        assert np.array_equal(p, _plan(L, M, N, K))
+
+
 def test_scales_are_pow2_predicate_and_cache():
     """The check that lets the MoE layers run the UE8M0 kernels under the
     FP32 contract: true only when every scale is a positive, finite, normal

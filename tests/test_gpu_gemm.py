@@ -904,3 +904,30 @@ def test_gemm_whole_line_store_paths(gpu_device, M, N, K, tile):
     assert_gemm_close(got, ref, f"store paths {M}x{N}x{K}")
     D1 = _gemm_gpu(qa[:M - 1], sa[:M - 1], qw, sw, gpu_device)
     assert np.array_equal(bf16_bits(D1), bf16_bits(D[:M - 1])), "rows depend on the row count"
+
+
+@pytest.mark.parametrize("M,N,K,tile", [(452, 200, 1024, (64, 64, 1)), (66, 200, 7168, (64, 64, 4)),
+                                        (194, 8200, 1024, (64, 256, 1)), (899, 200, 8192, (64, 256, 8)),
+                                        (200, 8192, 8192, (128, 64, 1)), (65, 3000, 8192, (128, 64, 5)),
+                                        (515, 7176, 1024, (128, 256, 1)), (129, 328, 4096, (128, 256, 8)),
+                                        (905, 8200, 1024, (192, 256, 1)), (2459, 3080, 1664, (256, 128, 1))])
+def test_gemm_dense_tile_choice(gpu_device, M, N, K, tile):
+    """Each tile the dense planner picks above 64 rows besides 128x128 and
+    256x256, whole and split over K, at ragged M and N: the NaN-prefilled
+    output is fully written and matches the oracle in every 64x64 block, and
+    packed per-row weight scales give the same bits."""
+    from kb_nano_amd import _ops
+    from tests._util import assert_all_written, tile_cover
+    p = _plan(M, N, K)
+    assert (p[0], p[1], p[5]) == tile, p
+    qa, sa, qw, sw = quantized_gemm_inputs(M, N, K, seed=M + 5 * N + K)
+    D = _gemm_gpu(qa, sa, qw, sw, gpu_device)
+    assert_all_written(D, f"{M}x{N}x{K}")
+    rows, cols = tile_cover(M, N, np.random.default_rng(M + N + K))
+    ref = oracle.gemm_nt_sample(qa, sa, qw, sw, rows=rows, cols=cols, ue8m0=True)
+    got = D[torch.from_numpy(rows).to(gpu_device)][:, torch.from_numpy(cols).to(gpu_device)]
+    assert_gemm_close(got, ref, f"dense tile {M}x{N}x{K}")
+    packed = _ops.pack_ue8m0_weight_scales(torch.from_numpy(sw).to(gpu_device), N, K)
+    D2 = torch.full((M, N), float("nan"), dtype=torch.bfloat16, device=gpu_device)
+    _ops.fp8_gemm_nt(to_fp8(qa, gpu_device), torch.from_numpy(sa).to(gpu_device), to_fp8(qw, gpu_device), packed, D2)
+    assert np.array_equal(bf16_bits(D), bf16_bits(D2)), "packed scales differ"
