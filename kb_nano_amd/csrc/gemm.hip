@@ -255,7 +255,7 @@ __global__ __launch_bounds__(256) void sorted_scale_gather_kernel(const GemmArgs
 
 // Sorted-token (fused MoE) launch: one workgroup per BM x BN tile of the
 // padded row grid; tiles past the padded total exit at once.
-template <int BM, int BN, int kStages>
+template <int BM, int BN, int kStages, int kWaves>
 static int launch_sorted(GemmArgs a, hipStream_t st, const char* what) {
     a.tiles_m = (a.M + BM - 1) / BM;
     a.tiles_n = (a.N + BN - 1) / BN;
@@ -269,7 +269,8 @@ static int launch_sorted(GemmArgs a, hipStream_t st, const char* what) {
     a.group_m = moe_group_m(a.K);
     const int64_t grid = moe_dealt_grid(a.tiles_m, a.tiles_n, a.group_m);
     KBN_CHECK_ARG(grid <= 0x7FFFFFFFLL, "%s: too many tiles", what);
-    gemm_bs_kernel<BM, BN, kStages, false, false, false, 4, true><<<dim3((unsigned)grid), dim3(256), 0, st>>>(a);
+    gemm_bs_kernel<BM, BN, kStages, false, false, false, kWaves, true>
+        <<<dim3((unsigned)grid), dim3(64 * kWaves), 0, st>>>(a);
     KBN_CHECK_LAUNCH(what);
     return 0;
 }
@@ -898,9 +899,15 @@ extern "C" int kbn_fp8_grouped_gemm_nt_contiguous(const void* A, int64_t lda, co
     // the expert's weight panel in L2.
     a.a_pad_zero = K <= kPadZeroMaxK;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    Schedule sc;   // grouped: data-parallel, one workgroup per 128-row block x N tile
-    if (scale_ue8m0) return launch_gemm<128, 256, 3, true, true>(a, sc, st, what);
-    return launch_gemm<128, 256, 3, false, true>(a, sc, st, what);
+    // grouped: data-parallel, one workgroup per 128-row block x N tile, of
+    // eight wavefronts: two per SIMD cover each other's waits, and the FP32
+    // contract's rescale is half as long per wavefront.  Experts layer, us,
+    // four -> eight (both GEMMs): 128 experts x 4096 x 1536, 515 tokens, scales
+    // as given 519 -> 484, 4096 tokens 1357 -> 1271; 256 x 7168 x 2048, 4096
+    // tokens 3253 -> 3129 as given, 2938 -> 2937 with powers of two.
+    Schedule sc;
+    if (scale_ue8m0) return launch_gemm<128, 256, 3, true, true, 8>(a, sc, st, what);
+    return launch_gemm<128, 256, 3, false, true, 8>(a, sc, st, what);
 }
 
 extern "C" int kbn_fp8_grouped_gemm_silu_quant(const void* A, int64_t lda, const float* sA, int64_t sA_stride_m,
@@ -946,8 +953,8 @@ extern "C" int kbn_fp8_grouped_gemm_silu_quant(const void* A, int64_t lda, const
     if (!a.silu_lut) return 1;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     Schedule sc;
-    if (scale_ue8m0) return launch_gemm<128, 256, 3, true, true, 4, 0, false, true>(a, sc, st, what);
-    return launch_gemm<128, 256, 3, false, true, 4, 0, false, true>(a, sc, st, what);
+    if (scale_ue8m0) return launch_gemm<128, 256, 3, true, true, 8, 0, false, true>(a, sc, st, what);
+    return launch_gemm<128, 256, 3, false, true, 8, 0, false, true>(a, sc, st, what);
 }
 
 extern "C" int64_t kbn_fp8_fused_moe_gemm_workspace_bytes(int64_t EM, int64_t K) {
@@ -1016,6 +1023,8 @@ extern "C" int kbn_fp8_fused_moe_gemm(const void* A, int64_t lda, int64_t rows_A
     }
     // the scales are taken as given (fp32 contract), as the reference's
     // per-block promotion does
-    if (block_m % 128 == 0) return launch_sorted<128, 256, 3>(a, st, what);
-    return launch_sorted<64, 256, 3>(a, st, what);
+    // eight wavefronts for 128-row blocks: VllmFusedExperts at 515 tokens 511 ->
+    // 503 us (128 experts x 4096 x 1536) and 1892 -> 1877 (256 x 7168 x 2048)
+    if (block_m % 128 == 0) return launch_sorted<128, 256, 3, 8>(a, st, what);
+    return launch_sorted<64, 256, 3, 4>(a, st, what);
 }

@@ -446,8 +446,8 @@ gemm_bs_kernel(const GemmArgs a) {
                               (kFuseA == 1 || kFuseA == 2 || kFuseA == 4)),
                   "in-kernel activation quant: UE8M0, dense, 64-row tiles of four wavefronts, 16/32/64 rows");
     static_assert(kWaves == 4 || kWaves == 8, "2x2 or 2x4 wavefronts");
-    static_assert(!kGlu || (kGrouped && BM == 128 && BN == 256 && kWaves == 4),
-                  "SiLU*Mul epilogue: the grouped 128x256 tiles (128 gate + 128 up columns, two per wavefront row)");
+    static_assert(!kGlu || (kGrouped && BM == 128 && BN == 256),
+                  "SiLU*Mul epilogue: the grouped 128x256 tiles (128 gate columns, then 128 up columns)");
     static_assert(!kRowW || (kUe8m0 && !kGrouped && !kSorted && !kFuseA && BN <= 64 * kWaves),
                   "packed per-row weight scales: dense UE8M0 tiles, one scale word per tile row and lane");
     constexpr int WM = 2, WN = kWaves / 2;
@@ -494,9 +494,18 @@ gemm_bs_kernel(const GemmArgs a) {
     const uint8_t* Wbase = a.W;
     const float* sWbase = a.sW;
     int expert = 0;
+    // Grouped: which of the tile's rows belong to its expert (the first row's),
+    // as two 64-row masks.  All 128 ids come in one round trip at the start;
+    // the epilogue and the padding checks below read the masks.  (Ids loaded
+    // where they were used, after the first row's and again in the epilogue,
+    // left each tile two more exposed load latencies.)
+    uint64_t live_lo = 0, live_hi = 0;
     if constexpr (kGrouped) {
-        expert = a.expert_ids[m0];
+        const int id0 = a.expert_ids[m0 + lane], id1 = a.expert_ids[m0 + 64 + lane];   // M is a multiple of 128
+        expert = __builtin_amdgcn_readfirstlane(id0);
         if (expert < 0 || expert >= a.E) return;  // padding block: C rows stay unwritten
+        live_lo = __ballot(id0 == expert);
+        live_hi = __ballot(id1 == expert);
         Wbase += (int64_t)expert * a.w_estride;
         sWbase += (int64_t)expert * a.sW_estride;
     }
@@ -508,6 +517,8 @@ gemm_bs_kernel(const GemmArgs a) {
         Wbase += (int64_t)expert * a.w_estride;
         sWbase += (int64_t)expert * a.sW_estride;
     }
+    // grouped: whether tile row r is one of the tile's expert
+    auto row_is_live = [&](int r) -> bool { return ((r < 64 ? live_lo : live_hi) >> (r & 63)) & 1; };
     // routed pair of tile row r, or -1 for padding
     auto pair_of = [&](int r) -> int {
         const int R = m0 + r;
@@ -535,7 +546,7 @@ gemm_bs_kernel(const GemmArgs a) {
     const int ch_o = ((lane & 7) ^ ((lane >> 4) | 4)) << 4;
     const int a_e = (int)((wave * kAInstr * 8 + drow) * a.lda) + ch_e + kb0 * kRowB;
     const int a_o = a_e - ch_e + ch_o;
-    // kGlu: the tile's W rows 128..255 (wavefronts 2 and 3) are the up rows,
+    // kGlu: the tile's W rows 128..255 (the upper half of the wavefronts) are the up rows,
     // glu_half - 128 rows further on than the tile's row index says
     const int glu_w = kGlu && wave * kBInstr * 8 >= BN / 2 ? (a.glu_half - BN / 2) * (int)a.ldw : 0;
     const int w_e = (int)((wave * kBInstr * 8 + drow) * a.ldw) + ch_e + kb0 * kRowB + glu_w;
@@ -559,8 +570,7 @@ gemm_bs_kernel(const GemmArgs a) {
         if (a.a_pad_zero) {
 #pragma unroll
             for (int i = 0; i < kAInstr; ++i) {
-                const int r = m0 + wave * kAInstr * 8 + i * 8 + drow;
-                if (r >= a.M || a.expert_ids[r] != expert) a_dead |= 1u << i;
+                if (!row_is_live(wave * kAInstr * 8 + i * 8 + drow)) a_dead |= 1u << i;
             }
         }
     }
@@ -648,33 +658,24 @@ gemm_bs_kernel(const GemmArgs a) {
     auto a_off = [&](int i) -> int { if constexpr (kKeepOff || kGrouped) return va[i]; else return a_voff(i); };
     auto w_off = [&](int i) -> int { if constexpr (kKeepOff) return vw[i]; else return w_voff(i); };
     int s_fetch = 0;   // the block to fetch next (0, with A and W unreadable, past the last)
-    // Load unit u (0 <= u < kUnits) of the block to fetch next, into stage S
-    // (a constant where the stages are unrolled): the scale vectors, then the
-    // A rows, then the W rows.
+    // Load unit u (0 <= u < kUnits) of the block to fetch next, into stage S:
+    // the scale vectors, then the A rows, then the W rows.
     auto issue_unit = [&](auto S_, auto u_) {
-        constexpr int u = decltype(u_)::value;
-        constexpr bool kConst = !std::is_same_v<decltype(S_), int>;
-        constexpr int S = [] { if constexpr (kConst) return (int)decltype(S_)::value; else return 0; }();
-        const int rt = kConst ? 0 : (int)S_;
+        constexpr int S = decltype(S_)::value, u = decltype(u_)::value;
         if constexpr (!kFuseA && u == 0) {
-            dma_b32<kOffS + S * (kSA + kSW)>(dSA, lds_s + rt * (kSA + kSW), sa_off0, s_fetch * sa_kstep);
+            dma_b32<kOffS + S * (kSA + kSW)>(dSA, lds_s, sa_off0, s_fetch * sa_kstep);
         } else if constexpr (u == kScaleDma - 1) {
-            dma_b32<kOffS + S * (kSA + kSW) + kSA>(dSW, lds_s + rt * (kSA + kSW), sw_off0,
+            dma_b32<kOffS + S * (kSA + kSW) + kSA>(dSW, lds_s, sw_off0,
                                                    kRowW ? ((kb0 + s_fetch) >> 2) * sw_kstep : s_fetch * sw_kstep);
         } else if constexpr (u < kScaleDma + kAUnits) {
             constexpr int i = (u - kScaleDma) * (kPairA ? 2 : 1);
             const int soff = s_fetch * (kFuseA ? 2 * kRowB : kRowB);
-            if constexpr (kPairA)
-                dma_b128_pair<S * kA + i * 1024, false>(dA, lds_a + rt * kA, a_off(i), a_off(i + 1), soff);
-            else
-                dma_b128<S * kA + i * 1024, false>(dA, lds_a + rt * kA, a_off(i), soff);
+            if constexpr (kPairA) dma_b128_pair<S * kA + i * 1024, false>(dA, lds_a, a_off(i), a_off(i + 1), soff);
+            else dma_b128<S * kA + i * 1024, false>(dA, lds_a, a_off(i), soff);
         } else {
-            constexpr int i = (u - kScaleDma - kAUnits) * (kPairW ? 2 : 1);
-            if constexpr (kPairW)
-                dma_b128_pair<kOffW + S * kB + i * 1024, kWeightNt>(dW, lds_w + rt * kB, w_off(i), w_off(i + 1),
-                                                                     s_fetch * kRowB);
-            else
-                dma_b128<kOffW + S * kB + i * 1024, kWeightNt>(dW, lds_w + rt * kB, w_off(i), s_fetch * kRowB);
+            constexpr int i = (u - kScaleDma - kAUnits) * (kPairW ? 2 : 1), off = kOffW + S * kB + i * 1024;
+            if constexpr (kPairW) dma_b128_pair<off, kWeightNt>(dW, lds_w, w_off(i), w_off(i + 1), s_fetch * kRowB);
+            else dma_b128<off, kWeightNt>(dW, lds_w, w_off(i), s_fetch * kRowB);
         }
     };
     // Past the last block the descriptors end at 0, so the A and W loads write
@@ -791,8 +792,7 @@ gemm_bs_kernel(const GemmArgs a) {
     if constexpr (kGrouped && !kUe8m0) {
 #pragma unroll
         for (int i = 0; i < FM; ++i) {
-            const int r = m0 + wm * TM + i * 32 + (lane & 31);
-            row_live[i] = r < a.M && a.expert_ids[r] == expert;
+            row_live[i] = row_is_live(wm * TM + i * 32 + (lane & 31));
         }
     }
     // E8M0 operands of raw scales (in the top byte); FP32 contract: the first block's mantissa
@@ -968,8 +968,7 @@ gemm_bs_kernel(const GemmArgs a) {
     int nlive = FM;
     if constexpr (kGrouped) {
         static_assert(!kGrouped || (FM == 2 && TM == 64), "one ballot bit per wavefront row, two A fragments");
-        const int r = m0 + wm * TM + lane;
-        const uint64_t live = __ballot(r < a.M && a.expert_ids[r] == expert);
+        const uint64_t live = wm ? live_hi : live_lo;
         nlive = (live >> 32) ? 2 : live ? 1 : 0;
     }
     auto want = [&](int q) { return !kGrouped || ((q >> 1) < FM ? (q >> 1) < nlive : nlive > 0); };
@@ -994,12 +993,9 @@ gemm_bs_kernel(const GemmArgs a) {
     // left to fetch.
     auto block = [&](auto S_, auto fetch_, int kb) {
         constexpr bool kFetch = decltype(fetch_)::value;
-        const int S = S_, next = S + 1 < kStages ? S + 1 : 0;
+        constexpr int S = decltype(S_)::value, next = (S + 1) % kStages;
         // blocks' loads issued after those of block kb+1
-        constexpr int kAhead = [] {
-            if constexpr (kFetch) return kStages - 2;
-            else return std::max(kStages - 2 - (int)decltype(S_)::value, 0);
-        }();
+        constexpr int kAhead = kFetch ? kStages - 2 : std::max(kStages - 2 - S, 0);
         rescale_all();
         // ---- sub-step 0: K half 0 of block kb; read K half 1
 #pragma unroll
@@ -1073,19 +1069,13 @@ gemm_bs_kernel(const GemmArgs a) {
     // instructions a block for a 128x64 tile's wavefront, 120 with the stage
     // computed).  us a call, stage computed -> unrolled: 8 x 10240 x 8192
     // 19.0 -> 17.4, 64 x 2048 x 2048 9.3 -> 8.9, 4096 x 36864 x 7168 836 ->
-    // 805.  The 128x256 MoE tiles stay as they were: in the larger loop the
-    // compiler moved their accumulators between register files (the experts
-    // layer 12% slower at 4096 tokens).
-    if constexpr (!((kGrouped || kSorted) && FM * FN >= 8)) {
-        int kb = 0;
-        for (; kb + kStages <= KB; kb += kStages)
-            static_for<kStages>([&](auto S_) { block(S_, std::true_type{}, kb + decltype(S_)::value); });
-        static_for<kStages - 1>([&](auto S_) {
-            if (kb + decltype(S_)::value < KB) block(S_, std::false_type{}, kb + decltype(S_)::value);
-        });
-    } else {
-        for (int kb = 0, st = 0; kb < KB; ++kb, st = st + 1 < kStages ? st + 1 : 0) block(st, std::true_type{}, kb);
-    }
+    // 805.
+    int kb = 0;
+    for (; kb + kStages <= KB; kb += kStages)
+        static_for<kStages>([&](auto S_) { block(S_, std::true_type{}, kb + decltype(S_)::value); });
+    static_for<kStages - 1>([&](auto S_) {
+        if (kb + decltype(S_)::value < KB) block(S_, std::false_type{}, kb + decltype(S_)::value);
+    });
     // the trailing (out-of-range) loads still target this workgroup's LDS
     wait_dma();
     if constexpr (!kUe8m0) {
@@ -1195,7 +1185,7 @@ gemm_bs_kernel(const GemmArgs a) {
         const int row = wm * TM + i * 32 + (lane & 31);
         if constexpr (kSorted) return out_row[i] >= 0 ? out_row[i] * (int)a.ldd * 2 : kOob;
         else if constexpr (kGrouped)
-            return (m0 + row < a.M && a.expert_ids[m0 + row] == expert) ? row * (int)a.ldd * 2 : kOob;
+            return row_is_live(row) ? row * (int)a.ldd * 2 : kOob;
         else return row * (int)a.ldd * 2;
     };
 
@@ -1266,26 +1256,29 @@ gemm_bs_kernel(const GemmArgs a) {
             if constexpr (kGrouped) {
                 static_assert(!kGrouped || TM <= 64, "one mask bit per wavefront row");
                 // kGlu: the rows of this wavefront's SiLU*Mul pass below
-                const int r = m0 + (kGlu ? wave * (BM / 4) : wm * TM) + lane;
-                row_mask = __ballot(lane < (kGlu ? BM / 4 : TM) && r < a.M && a.expert_ids[r] == expert);
+                constexpr int kGluRows = BM / kWaves;
+                if constexpr (kGlu) row_mask = (wave * kGluRows < 64 ? live_lo : live_hi) >> (wave * kGluRows & 63);
+                else row_mask = wm ? live_hi : live_lo;
             }
             wait_lds();
             if constexpr (kGlu) {
-                // SiLU*Mul + 1x128 quant: wavefront w takes tile rows [32 w, 32 w + 32),
-                // 16 lanes (one 128-column group) per row, four rows per pass;
-                // row rt's gate block is wavefront (rt / 64, 0)'s, its up block
-                // wavefront (rt / 64, 1)'s, both laid out as stored above
+                // SiLU*Mul + 1x128 quant: each wavefront takes BM / kWaves tile rows,
+                // 16 lanes (one 128-column group, 8 columns each) per row, four rows
+                // per pass; a row's gate columns lie in the blocks of the first half
+                // of its row's wavefronts, the up columns at the same place in the
+                // second half's, both laid out as stored above
                 __syncthreads();   // every wavefront's block is in LDS
                 const int sub = lane & 15, rq = lane >> 4;
 #pragma unroll
-                for (int it = 0; it < BM / 4 / 4; ++it) {
-                    const int rt = wave * (BM / 4) + it * 4 + rq;
+                for (int it = 0; it < BM / kWaves / 4; ++it) {
+                    const int rt = wave * (BM / kWaves) + it * 4 + rq;
                     const int r = m0 + rt;
                     if ((row_mask >> (it * 4 + rq)) & 1) {   // uniform over the row's 16 lanes
                         const int bw = rt / TM, rl = rt % TM;
-                        const uint8_t* gate = smem + (bw * WN) * (TM * kRowB2) + rl * kRowB2 + ((sub + rl) % kCh) * 16;
+                        const uint8_t* gate = smem + (bw * WN + sub / kCh) * (TM * kRowB2) + rl * kRowB2 +
+                                              ((sub % kCh + rl) % kCh) * 16;
                         const u32x4 g = *reinterpret_cast<const u32x4*>(gate);
-                        const u32x4 u = *reinterpret_cast<const u32x4*>(gate + TM * kRowB2);
+                        const u32x4 u = *reinterpret_cast<const u32x4*>(gate + WN / 2 * (TM * kRowB2));
                         const uint32_t w[4] = {silu_mul_pair(a.silu_lut, g.x, u.x), silu_mul_pair(a.silu_lut, g.y, u.y),
                                                silu_mul_pair(a.silu_lut, g.z, u.z), silu_mul_pair(a.silu_lut, g.w, u.w)};
                         uint8_t* q = a.q2 + (int64_t)r * a.ldq2 + n0;
