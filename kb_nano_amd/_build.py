@@ -73,6 +73,42 @@ def _compile(src: str, hipcc: str) -> str:
     return obj
 
 
+HOST_PATH = os.path.join(HERE, "_host.so")
+
+
+def _host_object() -> str:
+    """Compile ``csrc/host_calls.cpp`` (the eager host path of the small
+    calls, a CPython module over torch's C++ API) with the host compiler."""
+    import sysconfig
+
+    from torch.utils.cpp_extension import include_paths
+    cxx = shutil.which("g++") or shutil.which("c++")
+    if cxx is None:
+        raise RuntimeError("a host C++ compiler (g++) is needed to build the host calls")
+    src, obj = os.path.join(CSRC, "host_calls.cpp"), os.path.join(OBJ_DIR, "host_calls.cpp.o")
+    inc = [f"-I{p}" for p in [os.path.join(os.path.dirname(HERE), "include"), sysconfig.get_paths()["include"],
+                              *include_paths()]]
+    cmd = [cxx, "-O2", "-std=c++17", "-fPIC", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM=1", *inc,
+           "-isystem", "/opt/rocm/include", "-c", src, "-o", obj]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"building {src} failed:\n{' '.join(cmd)}\n{r.stderr[-4000:]}")
+    return obj
+
+
+def _link_host(obj: str) -> None:
+    """Link the host calls against the operator library next to them."""
+    import torch
+    lib_dir = os.path.join(os.path.dirname(torch.__file__), "lib")
+    tmp = HOST_PATH + ".tmp"
+    cmd = [shutil.which("g++") or "c++", "-shared", "-o", tmp, obj, "-L", HERE, f"-l:{LIB_NAME}", "-Wl,-rpath,$ORIGIN",
+           "-L", lib_dir, "-lc10", "-ltorch_cpu", "-ltorch_python", "-lc10_hip", "-L", "/opt/rocm/lib", "-lamdhip64"]
+    r = subprocess.run(cmd, capture_output=True, text=True)
+    if r.returncode != 0:
+        raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{r.stderr}")
+    os.replace(tmp, HOST_PATH)
+
+
 BENCH_CSRC = os.path.join(HERE, "bench_csrc")
 BENCH_LIB_PATH = os.path.join(HERE, "libkbn_bench.so")
 
@@ -102,14 +138,17 @@ def build(verbose: bool = False) -> str:
     sources = sorted(glob.glob(os.path.join(CSRC, "*.hip")))
     if not sources:
         raise RuntimeError(f"no HIP sources under {CSRC}")
-    with cf.ThreadPoolExecutor(max_workers=min(8, len(sources))) as ex:
+    with cf.ThreadPoolExecutor(max_workers=min(8, len(sources) + 1)) as ex:
+        host = ex.submit(_host_object)
         objs = list(ex.map(lambda s: _compile(s, hipcc), sources))
+        host_obj = host.result()
     tmp = LIB_PATH + ".tmp"
     cmd = [hipcc, f"--offload-arch={ARCH}", "-shared", "-fPIC", "-o", tmp, *objs]
     r = subprocess.run(cmd, capture_output=True, text=True)
     if r.returncode != 0:
         raise RuntimeError(f"link failed:\n{' '.join(cmd)}\n{r.stdout}\n{r.stderr}")
     os.replace(tmp, LIB_PATH)
+    _link_host(host_obj)
     build_bench(hipcc)
     if verbose:
         print(f"built {LIB_PATH} from {len(sources)} sources, and {BENCH_LIB_PATH}", file=sys.stderr)

@@ -23,6 +23,11 @@ import torch
 
 from ._lib import check, lib, require_gfx950
 
+try:   # the small calls' eager host path in one native step (csrc/host_calls.cpp)
+    from . import _host
+except ImportError:   # not built yet: the Python path makes the same launches
+    _host = None
+
 FP8 = torch.float8_e4m3fn
 GROUP = 128
 QUANT_EPS = 1e-10  # tasks/baseline/L1/fp8_linear.py:44

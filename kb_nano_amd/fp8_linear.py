@@ -117,6 +117,14 @@ class Fp8Linear(nn.Module):
 
     def forward(self, input_bf16: torch.Tensor, weight_fp8: torch.Tensor,
                 weight_scale_inv: torch.Tensor, bias: torch.Tensor | None = None) -> torch.Tensor:
+        if _ops._host is not None and not torch.compiler.is_compiling():
+            # bf16 rows, installed buffers: the choices below in one native
+            # step (1 x 2048 x 2048 9.2 -> 7.1 us a call, 200 x 2048 x 2048 13.1
+            # -> 10.2: host-bound before, the kernels now)
+            output = _ops._host.linear(input_bf16, weight_fp8, weight_scale_inv, self._a_buf, self._s_buf, self._o_buf,
+                                       self._pf, is_e8m0_used(), _ops._WS_BUFS)
+            if output is not None:
+                return output if bias is None else output + bias
         N, K = weight_fp8.shape
         in_shape = input_bf16.shape
         flat = len(in_shape) == 2 and in_shape[1] == K

