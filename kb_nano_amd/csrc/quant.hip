@@ -26,7 +26,8 @@
 //
 // SiLU: silu(g) of a bf16 g has only 65,536 possible inputs, so the fused
 // kernel reads bf16(silu(g)) (correctly rounded, generated at build time by
-// gen_silu_lut.cpp) from a 128 KB table staged in LDS, one table per CU.
+// gen_silu_lut.cpp) from a 128 KB table, staged in LDS for large inputs, one
+// table per CU.
 // y = bf16(silu * up) is the exact fp32 product rounded once by
 // v_cvt_pk_bf16_f32.
 
@@ -52,6 +53,17 @@ typedef short s16x2 __attribute__((ext_vector_type(2)));
 #define KBN_QUANT_PER_CU 2
 #endif
 constexpr int kThreads = 1024;       // 16 wavefronts
+// Small workgroups (four wavefronts, one block each a pass, up to 8 a CU): the
+// bf16 quant always, the SiLU kernel up to kSmallSiluGroups groups.  A launch
+// of 16-wavefront workgroups ramps up slower: quant, us in a graph, large ->
+// small: 64 x 2048 2.85 -> 2.10, 200 x 7168 3.58 -> 2.72, 777 x 7168 5.77 ->
+// 5.19, 8192 x 7168 31.8 -> 31.5, 4096 x 18432 40.0 -> 40.1.  The SiLU kernel
+// also copies its 128 KB table into each CU's LDS, which only many groups
+// repay: 128 x 2048 6.17 -> 2.53, 400 x 7168 8.13 -> 6.75, 200 x 18432 (28,800
+// groups) 8.81 -> 7.88, but 777 x 7168 (43,512) 9.62 -> 10.93 and
+// 8192 x 18432 135 -> 188.
+constexpr int kSmallThreads = 256;
+constexpr int64_t kSmallSiluGroups = 32768;
 // 4-group blocks per wavefront per pass (per operand): the SiLU kernel runs
 // one workgroup per CU (its LDS table), so it takes more blocks per pass to
 // keep as many bytes in flight (measured at cfg2: 4 -> 129 us, 2 -> 132 us,
@@ -161,14 +173,19 @@ __device__ __forceinline__ float quant8f_store(const float (&v)[8], float eps, i
 // XCDs in blocks of 32 (block b to XCD b % 8) instead of contiguous slices:
 // skipped rows cluster (an expert segment's padding, the layout's unused
 // tail), and contiguous slices would leave whole XCDs without work.
-template <bool kSilu, bool kUe8m0, bool kRows = false, int kIn = kInBf16>
-__global__ __launch_bounds__(kThreads) void group_quant_kernel(const QuantArgs a) {
+// kSmall: workgroups of four wavefronts instead of 16, one block per
+// wavefront and pass, and no SiLU table in LDS (read where it lies, from L2).
+template <bool kSilu, bool kUe8m0, bool kRows = false, int kIn = kInBf16, bool kSmall = false>
+__global__ __launch_bounds__(kSmall ? kSmallThreads : kThreads) void group_quant_kernel(const QuantArgs a) {
+    constexpr int kThreads = kSmall ? kSmallThreads : kbn::kThreads;
+    constexpr bool kTable = kSilu && !kSmall;
     static_assert(kIn == kInBf16 || (!kSilu && !kRows), "the SiLU and row-skipping kernels take bf16 input");
     constexpr int kEb = kIn == kInF32 ? 4 : 2;   // input bytes per element
-    __shared__ __attribute__((aligned(16))) uint16_t lut[kSilu ? 65536 : 8];
-    if constexpr (kSilu) {  // stage the bf16 SiLU table: 8192 x 16 B
+    __shared__ __attribute__((aligned(16))) uint16_t table[kTable ? 65536 : 8];
+    const uint16_t* const lut = kTable ? table : kSiluLut;
+    if constexpr (kTable) {  // stage the bf16 SiLU table: 8192 x 16 B
         const u32x4* src = reinterpret_cast<const u32x4*>(kSiluLut);
-        u32x4* dst = reinterpret_cast<u32x4*>(lut);
+        u32x4* dst = reinterpret_cast<u32x4*>(table);
 #pragma unroll
         for (int i = 0; i < 8192 / kThreads; ++i) dst[threadIdx.x + i * kThreads] = src[threadIdx.x + i * kThreads];
         __syncthreads();
@@ -180,7 +197,7 @@ __global__ __launch_bounds__(kThreads) void group_quant_kernel(const QuantArgs a
     const int row_begin = kRows ? 0 : xcd * a.rows_per_xcd;
     const int row_end = kRows ? a.rows_per_xcd : min(a.M, row_begin + a.rows_per_xcd);
     auto grow = [&](int lr) { return kRows ? (((lr >> 5) * kXcds + xcd) << 5) + (lr & 31) : lr; };
-    constexpr int kUnroll = kUnrollOf<kSilu>;
+    constexpr int kUnroll = kSmall ? 1 : kUnrollOf<kSilu>;
     const int64_t t0 = ((int64_t)local * (kThreads / 64) + wave) * (4 * kUnroll) + (lane >> 4);
     GroupCursor c{row_begin + (int)(t0 / a.G), (int)(t0 % a.G)};
     // kRows: the row ids of the groups of the next pass, loaded one pass
@@ -300,10 +317,10 @@ __global__ void silu_bf16_debug_kernel(const uint16_t* __restrict__ g, uint16_t*
 
 // Row slices per XCD (multiples of 32 rows) and the number of workgroups
 // per XCD: at most `per_cu` per CU, never more than the slice needs.
-static int plan(QuantArgs& a, int per_cu, int unroll) {
+static int plan(QuantArgs& a, int per_cu, int unroll, int threads = kThreads) {
     const int slice = (a.M + kXcds - 1) / kXcds;
     a.rows_per_xcd = (slice + kLineRows - 1) / kLineRows * kLineRows;
-    const int64_t per_block = (int64_t)(kThreads / 64) * 4 * unroll;  // groups per workgroup pass
+    const int64_t per_block = (int64_t)(threads / 64) * 4 * unroll;  // groups per workgroup pass
     const int64_t need = ((int64_t)a.rows_per_xcd * a.G + per_block - 1) / per_block;
     const int per_xcd = (int)std::max<int64_t>(1, std::min<int64_t>(need, (int64_t)cu_count() / kXcds * per_cu));
     const int64_t stride = (int64_t)per_xcd * per_block;
@@ -341,12 +358,16 @@ static int quant_typed(const char* what, const void* x, int x_dtype, int64_t M, 
     KBN_CHECK_ARG(ld_x >= K, "%s: input row stride smaller than K", what);
     QuantArgs a{(const uint16_t*)x, ld_x, 0, (uint8_t*)q_fp8, ld_q, scale, s_stride_m, s_stride_g,
                 (int)M, (int)(K / kGroup), 0, 0, 0, eps};
-    const int blocks = plan(a, KBN_QUANT_PER_CU, kUnrollOf<false>);
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     if (x_dtype == kInBf16) {
-        if (use_ue8m0) group_quant_kernel<false, true><<<blocks, kThreads, 0, st>>>(a);
-        else group_quant_kernel<false, false><<<blocks, kThreads, 0, st>>>(a);
-    } else if (x_dtype == kInF16) {
+        const int blocks = plan(a, 8, 1, kSmallThreads);
+        if (use_ue8m0) group_quant_kernel<false, true, false, kInBf16, true><<<blocks, kSmallThreads, 0, st>>>(a);
+        else group_quant_kernel<false, false, false, kInBf16, true><<<blocks, kSmallThreads, 0, st>>>(a);
+        KBN_CHECK_LAUNCH(what);
+        return 0;
+    }
+    const int blocks = plan(a, KBN_QUANT_PER_CU, kUnrollOf<false>);
+    if (x_dtype == kInF16) {
         if (use_ue8m0) group_quant_kernel<false, true, false, kInF16><<<blocks, kThreads, 0, st>>>(a);
         else group_quant_kernel<false, false, false, kInF16><<<blocks, kThreads, 0, st>>>(a);
     } else {
@@ -380,8 +401,15 @@ extern "C" int kbn_silu_mul_quant_fp8(const void* in_bf16, int64_t M, int64_t N_
     KBN_CHECK_ARG(ld_in >= 2 * N_half, "%s: input row stride smaller than 2*N/2", what);
     QuantArgs a{(const uint16_t*)in_bf16, ld_in, N_half, (uint8_t*)q_fp8, ld_q, scale, s_stride_m, s_stride_g,
                 (int)M, (int)(N_half / kGroup), 0, 0, 0, eps};
-    const int blocks = plan(a, 1, kUnrollOf<true>);  // the LDS table allows one workgroup per CU
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
+    if (M * a.G <= kSmallSiluGroups) {
+        const int blocks = plan(a, 8, 1, kSmallThreads);
+        if (use_ue8m0) group_quant_kernel<true, true, false, kInBf16, true><<<blocks, kSmallThreads, 0, st>>>(a);
+        else group_quant_kernel<true, false, false, kInBf16, true><<<blocks, kSmallThreads, 0, st>>>(a);
+        KBN_CHECK_LAUNCH(what);
+        return 0;
+    }
+    const int blocks = plan(a, 1, kUnrollOf<true>);  // the LDS table allows one workgroup per CU
     if (use_ue8m0)
         group_quant_kernel<true, true><<<blocks, kThreads, 0, st>>>(a);
     else

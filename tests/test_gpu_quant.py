@@ -355,3 +355,29 @@ def test_silu_mul_quant_nonfinite(gpu_device):
     torch.cuda.synchronize()
     assert np.array_equal(s.cpu().numpy(), so)
     assert np.array_equal(_canon_nan(fp8_codes(q)), _canon_nan(qo))
+
+
+@pytest.mark.parametrize("M,Nh", [(256, 128 * 127), (256, 128 * 128), (256, 128 * 129), (1, 128), (5, 384)])
+@pytest.mark.parametrize("use_ue8m0", [True, False])
+def test_silu_mul_quant_table_in_lds_or_not(gpu_device, M, Nh, use_ue8m0):
+    """The SiLU kernel reads its table where it lies up to 32,768 groups and
+    from LDS beyond; both sides of that line and the smallest sizes, with
+    infinities and NaN, against the oracle."""
+    x = seeded_bf16((M, 2 * Nh), seed=M + Nh).float().numpy()
+    x[0, 3], x[M // 2, 100], x[M - 1, 7], x[M - 1, Nh + 9] = np.inf, -np.inf, np.nan, np.nan
+    bits = oracle.f32_to_bf16_bits(x)
+    qo, so = oracle.silu_mul_quant(bits, use_ue8m0=use_ue8m0)
+    q, s = _silu_gpu(from_bits(bits, gpu_device), use_ue8m0=use_ue8m0)
+    assert np.array_equal(s.cpu().numpy(), so, equal_nan=True)
+    assert np.array_equal(_canon_nan(fp8_codes(q)), _canon_nan(qo))
+
+
+@pytest.mark.parametrize("M,K", [(1, 128), (1, 640), (33, 384), (257, 1152), (300, 7168), (2049, 2048)])
+def test_quant_workgroup_edges(gpu_device, M, K):
+    """Group counts around a wavefront's four, a workgroup's sixteen and the
+    XCDs' 32-row slices, row- and column-major scales."""
+    x = seeded_bf16((M, K), seed=M + K, outlier_frac=1e-3)
+    qo, so = oracle.quant_group128(bf16_bits(x))
+    for col_major in (False, True):
+        q, s = _quant_gpu(x.to(gpu_device), col_major=col_major)
+        assert np.array_equal(s.cpu().numpy(), so) and np.array_equal(fp8_codes(q), qo)
