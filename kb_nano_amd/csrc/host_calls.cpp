@@ -63,18 +63,19 @@ at::Tensor empty_scales(const at::Tensor& like, int64_t rows, int64_t groups) { 
 }
 
 // An eager workspace of at least `bytes` for (device, stream), from the dict
-// the Python side keeps ({(device, stream): uint8 tensor}); nullptr if it has
-// none that large.
-void* kept_workspace(PyObject* bufs, int64_t dev, hipStream_t st, int64_t bytes) {
+// the Python side keeps ({(device, stream): uint8 tensor}); undefined if it
+// has none that large.  The caller holds the tensor over its launch: another
+// thread may put a larger one in its place once the GIL is released.
+at::Tensor kept_workspace(PyObject* bufs, int64_t dev, hipStream_t st, int64_t bytes) {
     PyObject* key = Py_BuildValue("(LL)", (long long)dev, (long long)(intptr_t)st);
     if (!key) {
         PyErr_Clear();
-        return nullptr;
+        return {};
     }
     PyObject* buf = PyDict_GetItem(bufs, key);   // borrowed; no exception set
     Py_DECREF(key);
     const at::Tensor* t = buf ? plain_tensor(buf) : nullptr;
-    return t && t->numel() >= bytes ? t->data_ptr() : nullptr;
+    return t && t->numel() >= bytes ? *t : at::Tensor();
 }
 
 // Failures of the torch calls (out of memory, say) surface from the Python path.
@@ -200,12 +201,14 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
         if (!o || !is(*o, at::kBFloat16, dev, 2) || o->size(0) < M || o->size(1) != N || o->stride(1) != 1) Py_RETURN_NONE;
         int rc;
         if (direct) {
-            void* wsp = direct->ws ? kept_workspace(args[8], dev, st, direct->ws) : nullptr;
-            if (direct->ws && !wsp) Py_RETURN_NONE;
+            const int64_t bytes = direct->ws;
+            const at::Tensor buf = bytes ? kept_workspace(args[8], dev, st, bytes) : at::Tensor();
+            if (bytes && !buf.defined()) Py_RETURN_NONE;
+            void* const wsp = bytes ? buf.data_ptr() : nullptr;
             Py_BEGIN_ALLOW_THREADS
             rc = kbn_fp8_gemm_bf16a(x->data_ptr(), x->stride(0), kQuantEps, w->data_ptr(), w->stride(0),
                                     (const float*)ws->data_ptr(), ws->stride(0), o->data_ptr(), o->stride(0), M, N, K, wsp,
-                                    direct->ws, (void*)st);
+                                    bytes, (void*)st);
             Py_END_ALLOW_THREADS
         } else {
             const at::Tensor *q = plain_tensor(qo), *s = plain_tensor(so);
@@ -213,8 +216,9 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
                 q->size(1) != K || q->stride(1) != 1 || s->size(0) < M || s->size(1) != K / kGroup)
                 Py_RETURN_NONE;
             const int64_t bytes = kbn_fp8_gemm_nt_workspace_bytes(M, N, K, ue8m0);
-            void* wsp = bytes ? kept_workspace(args[8], dev, st, bytes) : nullptr;
-            if (bytes && !wsp) Py_RETURN_NONE;
+            const at::Tensor buf = bytes ? kept_workspace(args[8], dev, st, bytes) : at::Tensor();
+            if (bytes && !buf.defined()) Py_RETURN_NONE;
+            void* const wsp = bytes ? buf.data_ptr() : nullptr;
             Py_BEGIN_ALLOW_THREADS
             rc = kbn_fp8_linear_forward(x->data_ptr(), M, K, x->stride(0), q->data_ptr(), q->stride(0),
                                         (float*)s->data_ptr(), s->stride(0), s->stride(1), kQuantEps, 1, w->data_ptr(),
