@@ -20,7 +20,7 @@
 //    product multiplies the sum before the store.  Power-of-two scales give
 //    ratios of 1 and skip the rescale, so such scales cost what UE8M0 does.
 //
-// Dataflow per workgroup (256 lanes = 4 wavefronts, one per SIMD):
+// Dataflow per workgroup (256 lanes = 4 wavefronts, one per SIMD; or 8, two per SIMD):
 //   HBM --buffer_load_dwordx4 ... lds (direct DMA)--> LDS (kStages x (BM+BN) x 128 B)
 //   LDS --ds_read_b128--> VGPR fragments --MFMA 32x32x64--> fp32 accumulators
 // Each LDS row is 128 B (one 128-K scale block); its eight 16-B chunks are
@@ -401,7 +401,8 @@ constexpr int gemm_occupancy(int bm, int bn, int stages, int fuse_a = 0) {
 }
 
 // Block-scaled GEMM tile kernel: BM x BN output tile, four wavefronts in a
-// 2 x 2 grid, each owning a (BM/2) x (BN/2) block of 32x32 MFMA fragments.
+// 2 x 2 grid (eight in 2 x 4), each owning a (BM/2) x (BN/2) (BN/4) block of
+// 32x32 MFMA fragments.
 //
 // LDS layout, operand by operand (one stage = one 128-K block):
 //   kStages x [A: BM x 128 B], kStages x [W: BN x 128 B], kStages x [sA: 4 x 64 fp32][sW: 4 x 64 fp32]
@@ -616,8 +617,8 @@ gemm_bs_kernel(const GemmArgs a) {
     constexpr int kScaleDma = kFuseA ? 1 : 2;    // scale vectors per stage (no A scales when fused)
     constexpr int kDma = kAInstr + kBInstr + kScaleDma;  // DMA instructions per wave per stage
     // Weight rows stream past L2 (non-temporal) where the weights dominate the
-    // traffic: the 128-column dense tiles (chosen only for M <= 128) and the
-    // grouped and sorted MoE tiles.  The large dense tiles keep the default,
+    // traffic: the 128-column dense tiles (above 128 rows the planner's prices
+    // hold it) and the grouped and sorted MoE tiles.  The large dense tiles keep the default,
     // which measures faster where A and W tiles are both re-read from L2.
     constexpr bool kWeightNt = (BN == 128) || kGrouped || kSorted;
 
