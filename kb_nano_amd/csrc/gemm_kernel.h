@@ -161,32 +161,35 @@ __device__ __forceinline__ v4i make_desc(const void* base, int64_t bytes) {
 // at least 8 rows of 128 bytes in).  kNt: the weight rows of a tile are read
 // once per workgroup and should not push the activation rows (read by every
 // workgroup of a tile row) out of L2.
+// The s_nop: a direct LDS load needs one wait state after a scalar write of
+// M0, and the compiler, which puts it in around its own instructions, does not
+// look inside the asm (tests/test_wait_states.py reads the built code).
 template <int kOff>
 __device__ __forceinline__ void dma_b32(const v4i& desc, uint32_t base, int voff, int soff) {
-    asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dword %2, %3, %4 offen lds" ::"s"(base), "n"(kOff), "v"(voff),
+    asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dword %2, %3, %4 offen lds" ::"s"(base), "n"(kOff), "v"(voff),
                  "s"(desc), "s"(soff)
                  : "memory", "scc");
 }
 template <int kOff, bool kNt>
 __device__ __forceinline__ void dma_b128(const v4i& desc, uint32_t base, int voff, int soff) {
     if constexpr (kNt)
-        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds" ::"s"(base), "n"(kOff),
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen nt lds" ::"s"(base), "n"(kOff),
                      "v"(voff), "s"(desc), "s"(soff)
                      : "memory", "scc");
     else
-        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" ::"s"(base), "n"(kOff),
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %3, %4 offen lds" ::"s"(base), "n"(kOff),
                      "v"(voff), "s"(desc), "s"(soff)
                      : "memory", "scc");
 }
 template <int kOff, bool kNt>
 __device__ __forceinline__ void dma_b128_pair(const v4i& desc, uint32_t base, int v0, int v1, int soff) {
     if constexpr (kNt)
-        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %4, %5 offen nt lds\n\t"
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, %5 offen nt lds\n\t"
                      "buffer_load_dwordx4 %3, %4, %5 offen offset:1024 nt lds" ::"s"(base),
                      "n"(kOff), "v"(v0), "v"(v1), "s"(desc), "s"(soff)
                      : "memory", "scc");
     else
-        asm volatile("s_add_u32 m0, %0, %1\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
+        asm volatile("s_add_u32 m0, %0, %1\n\ts_nop 0\n\tbuffer_load_dwordx4 %2, %4, %5 offen lds\n\t"
                      "buffer_load_dwordx4 %3, %4, %5 offen offset:1024 lds" ::"s"(base),
                      "n"(kOff), "v"(v0), "v"(v1), "s"(desc), "s"(soff)
                      : "memory", "scc");
