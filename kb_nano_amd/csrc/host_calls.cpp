@@ -4,9 +4,10 @@
 // the module's tensors, makes the checks, allocates the outputs and calls the
 // C entry point in one step; whatever is not the plain case (another type,
 // layout or device, a tensor subclass, an active mode or transform, graph
-// capture, a workspace that must grow, an argument the entry point refuses)
-// returns None and the caller takes its Python path, which handles it or
-// raises.  Figures stand at the callers.
+// capture, a workspace that must grow, an argument the entry point refuses
+// before it launches anything) returns None and the caller takes its Python
+// path, which handles it or raises.  An error after a launch raises here: the
+// call is never made a second time.  Figures stand at the callers.
 #include <Python.h>
 
 #include <ATen/ATen.h>
@@ -16,6 +17,8 @@
 #include <c10/hip/HIPFunctions.h>
 #include <c10/hip/HIPStream.h>
 #include <torch/csrc/autograd/python_variable.h>
+
+#include <utility>
 
 #include "kbn_fp8.h"
 
@@ -89,6 +92,42 @@ PyObject* guarded(F&& f) {
     }
 }
 
+// What a call that ended with `rc` != 0 gives.  1: an argument was refused and
+// nothing was launched, so None, and the Python path refuses it too.  Anything
+// else comes after a launch (the runtime's last error, which may be another
+// call's): the launch may have run, and a fused add + norm run again would add
+// twice, so the error is raised as the Python path raises it.
+PyObject* failed(int rc, const char* what) {
+    if (rc == 1) Py_RETURN_NONE;
+    if (PyObject* lib = PyImport_ImportModule("kb_nano_amd._lib")) {
+        PyObject* r = PyObject_CallMethod(lib, "check", "is", rc, what);   // raises KbnError
+        Py_DECREF(lib);
+        Py_XDECREF(r);
+    }
+    if (!PyErr_Occurred()) PyErr_Format(PyExc_RuntimeError, "%s failed (code %d)", what, rc);
+    return nullptr;
+}
+
+// failed(code, name): the rule above, for tests
+PyObject* failed_call(PyObject*, PyObject* const* args, Py_ssize_t n) {
+    const char* what = n == 2 ? PyUnicode_AsUTF8(args[1]) : nullptr;
+    const long rc = what ? PyLong_AsLong(args[0]) : 0;
+    if (!what || PyErr_Occurred()) return PyErr_Format(PyExc_TypeError, "failed(code, name)");
+    return failed((int)rc, what);
+}
+
+// (codes, scales), made before the launch so that nothing but the launch can
+// fail after it; empty with the Python error set if it cannot be made.
+struct Ref {
+    PyObject* p;
+    ~Ref() { Py_XDECREF(p); }
+    PyObject* take() { return std::exchange(p, nullptr); }
+};
+PyObject* pair(const at::Tensor& q, const at::Tensor& s) {
+    Ref a{THPVariable_Wrap(q)}, b{THPVariable_Wrap(s)};
+    return a.p && b.p ? PyTuple_Pack(2, a.p, b.p) : nullptr;
+}
+
 // norm(input, weight, eps, residual | None) -> (codes, scales) | None
 PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
     if (n != 4) Py_RETURN_NONE;
@@ -106,14 +145,16 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                         r->sizes() != x->sizes())))
             Py_RETURN_NONE;
         const at::Tensor q = empty_codes(*x, T, H), s = empty_scales(*x, T, (H + kGroup - 1) / kGroup);
+        Ref out{pair(q, s)};
+        if (!out.p) return nullptr;
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = kbn_rmsnorm_fp8_quant(x->data_ptr(), T, H, H, w->data_ptr(), add ? r->data_ptr() : nullptr, H, q.data_ptr(),
                                    H, (float*)s.data_ptr(), s.stride(0), s.stride(1), (float)PyFloat_AS_DOUBLE(args[2]),
                                    (void*)st);
         Py_END_ALLOW_THREADS
-        if (rc) Py_RETURN_NONE;
-        return Py_BuildValue("(NN)", THPVariable_Wrap(q), THPVariable_Wrap(s));
+        if (rc) return failed(rc, add ? "fused_add_rmsnorm_fp8_quant" : "rmsnorm_fp8_quant");
+        return out.take();
     });
 }
 
@@ -130,14 +171,16 @@ PyObject* silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const int64_t M = x->size(0), Nh = x->size(1) / 2;
         if (M % kGroup || Nh % kGroup || x->size(1) % 2) Py_RETURN_NONE;
         const at::Tensor q = empty_codes(*x, M, Nh), s = empty_scales(*x, M, Nh / kGroup);
+        Ref out{pair(q, s)};
+        if (!out.p) return nullptr;
         const int ue8m0 = PyObject_IsTrue(args[1]);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = kbn_silu_mul_quant_fp8(x->data_ptr(), M, Nh, x->stride(0), q.data_ptr(), Nh, (float*)s.data_ptr(), s.stride(0),
                                     s.stride(1), (float)PyFloat_AS_DOUBLE(args[2]), ue8m0, (void*)st);
         Py_END_ALLOW_THREADS
-        if (rc) Py_RETURN_NONE;
-        return Py_BuildValue("(NN)", THPVariable_Wrap(q), THPVariable_Wrap(s));
+        if (rc) return failed(rc, "silu_mul_quant_fp8");
+        return out.take();
     });
 }
 
@@ -226,7 +269,7 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
                                         o->stride(0), N, ue8m0, wsp, bytes, (void*)st);
             Py_END_ALLOW_THREADS
         }
-        if (rc) Py_RETURN_NONE;
+        if (rc) return failed(rc, direct ? "fp8_gemm_bf16a" : "fp8_linear_forward");
         if (o->size(0) == M) {
             Py_INCREF(oo);
             return oo;
@@ -239,6 +282,7 @@ PyMethodDef kMethods[] = {
     {"norm", (PyCFunction)(void (*)())norm, METH_FASTCALL, "RMSNorm (+ residual add) + 1x128 quant"},
     {"silu", (PyCFunction)(void (*)())silu, METH_FASTCALL, "SiLU*Mul + 1x128 quant"},
     {"linear", (PyCFunction)(void (*)())linear, METH_FASTCALL, "bf16 activations through an FP8 weight"},
+    {"failed", (PyCFunction)(void (*)())failed_call, METH_FASTCALL, "what a call gives for an error code"},
     {nullptr, nullptr, 0, nullptr},
 };
 PyModuleDef kModule = {PyModuleDef_HEAD_INIT, "_host", nullptr, -1, kMethods, nullptr, nullptr, nullptr, nullptr};

@@ -733,3 +733,17 @@ def test_scales_are_pow2_predicate_and_cache():
         assert _ops.scales_are_pow2(w)          # not seen: documented
         _ops._SCALE_WRITES[0] += 1
         assert not _ops.scales_are_pow2(w)
+
+
+def test_native_step_never_repeats_a_launch():
+    """The native host step leaves a call to the Python path, which makes it
+    again, only for code 1 (refused before any launch); any other code comes
+    after a launch (a fused add + norm has then updated its operands in place)
+    and is raised as the Python path raises it."""
+    from kb_nano_amd import _ops
+    from kb_nano_amd._lib import KbnError, lib
+    assert _ops._host.failed(1, "norm") is None
+    lib().kbn_debug_gemm_plan(0, 0, 0, 0, 0, None)   # leaves a message
+    for code in (2, -1, 700):
+        with pytest.raises(KbnError, match=rf"norm: debug_gemm_plan: bad arguments \(code {code}\)"):
+            _ops._host.failed(code, "norm")

@@ -1,6 +1,8 @@
 """The native host path of the small calls (csrc/host_calls.cpp) against the
 Python path it stands for: the same bytes, and None (so the Python path) for
 everything but the plain case."""
+import ctypes
+
 import pytest
 import torch
 
@@ -106,3 +108,31 @@ def test_anything_but_the_plain_case_is_left_to_python(gpu_device):
         RMSNormFP8Quant()(x, w[:128])
     with pytest.raises(AssertionError):
         SiluMulQuantFp8()(y[:100])
+
+
+def _leave_an_error():
+    """An error of an earlier runtime call on this thread, still unread: a
+    device index that does not exist, refused by the runtime on the host."""
+    with open("/proc/self/maps") as f:
+        hip = next(line.split()[-1] for line in f if "libamdhip64" in line)
+    assert ctypes.CDLL(hip).hipSetDevice(9999) != 0
+
+
+@pytest.mark.parametrize("native", [True, False])
+def test_a_pending_error_does_not_repeat_the_call(gpu_device, monkeypatch, native):
+    """An error left pending is reported after the launch: the call raises, as
+    the Python path does, and the operands were updated once, not twice."""
+    from kb_nano_amd._lib import KbnError
+    g = torch.Generator(device=gpu_device).manual_seed(3)
+    x, r = (torch.randn(61, 2048, device=gpu_device, generator=g).to(BF16) for _ in range(2))
+    w = torch.randn(2048, device=gpu_device, generator=g).to(BF16)
+    x1, r1 = x.clone(), r.clone()
+    FusedAddRMSNormFP8Quant()(x1, r1, w)
+    torch.cuda.synchronize()
+    if not native:
+        monkeypatch.setattr(_ops, "_host", None)
+    _leave_an_error()
+    with pytest.raises(KbnError, match="launch failed"):
+        FusedAddRMSNormFP8Quant()(x, r, w)
+    torch.cuda.synchronize()
+    assert torch.equal(r, r1) and torch.equal(x, x1)
