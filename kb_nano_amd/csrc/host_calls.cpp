@@ -164,6 +164,8 @@ PyObject* silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
     return guarded([&]() -> PyObject* {
         const at::Tensor* x = plain_tensor(args[0]);
         if (!x || !PyFloat_CheckExact(args[2]) || !plain_thread()) Py_RETURN_NONE;
+        const int ue8m0 = PyObject_IsTrue(args[1]);   // any object, as in Python: its truth value may raise
+        if (ue8m0 < 0) return nullptr;
         const int64_t dev = x->get_device();
         hipStream_t st;
         if (!is(*x, at::kBFloat16, dev, 2) || x->numel() == 0 || x->stride(1) != 1 || !launch_stream(dev, st))
@@ -173,7 +175,6 @@ PyObject* silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
         const at::Tensor q = empty_codes(*x, M, Nh), s = empty_scales(*x, M, Nh / kGroup);
         Ref out{pair(q, s)};
         if (!out.p) return nullptr;
-        const int ue8m0 = PyObject_IsTrue(args[1]);
         int rc;
         Py_BEGIN_ALLOW_THREADS
         rc = kbn_silu_mul_quant_fp8(x->data_ptr(), M, Nh, x->stride(0), q.data_ptr(), Nh, (float*)s.data_ptr(), s.stride(0),

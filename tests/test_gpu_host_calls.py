@@ -136,3 +136,14 @@ def test_a_pending_error_does_not_repeat_the_call(gpu_device, monkeypatch, nativ
         FusedAddRMSNormFP8Quant()(x, r, w)
     torch.cuda.synchronize()
     assert torch.equal(r, r1) and torch.equal(x, x1)
+
+
+def test_a_flag_without_a_truth_value(gpu_device):
+    """``use_ue8m0`` may be any object; the error its truth value raises comes out as it is."""
+    class Bad:
+        def __bool__(self):
+            raise ZeroDivisionError("no truth value")
+    x = torch.ones(128, 512, device=gpu_device, dtype=BF16)
+    with pytest.raises(ZeroDivisionError, match="no truth value"):
+        SiluMulQuantFp8()(x, use_ue8m0=Bad())
+    _same(SiluMulQuantFp8()(x, use_ue8m0=[]), SiluMulQuantFp8()(x, use_ue8m0=False))
