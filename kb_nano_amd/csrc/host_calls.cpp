@@ -81,6 +81,13 @@ at::Tensor kept_workspace(PyObject* bufs, int64_t dev, hipStream_t st, int64_t b
     return t && t->numel() >= bytes ? *t : at::Tensor();
 }
 
+// No GIL while it lives; taken again on every way out, an exception included
+// (guarded below calls into Python).
+struct NoGil {
+    PyThreadState* s = PyEval_SaveThread();
+    ~NoGil() { PyEval_RestoreThread(s); }
+};
+
 // Failures of the torch calls (out of memory, say) surface from the Python path.
 template <class F>
 PyObject* guarded(F&& f) {
@@ -148,11 +155,12 @@ PyObject* norm(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Ref out{pair(q, s)};
         if (!out.p) return nullptr;
         int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = kbn_rmsnorm_fp8_quant(x->data_ptr(), T, H, H, w->data_ptr(), add ? r->data_ptr() : nullptr, H, q.data_ptr(),
-                                   H, (float*)s.data_ptr(), s.stride(0), s.stride(1), (float)PyFloat_AS_DOUBLE(args[2]),
-                                   (void*)st);
-        Py_END_ALLOW_THREADS
+        {
+            NoGil no_gil;
+            rc = kbn_rmsnorm_fp8_quant(x->data_ptr(), T, H, H, w->data_ptr(), add ? r->data_ptr() : nullptr, H, q.data_ptr(),
+                                       H, (float*)s.data_ptr(), s.stride(0), s.stride(1), (float)PyFloat_AS_DOUBLE(args[2]),
+                                       (void*)st);
+        }
         if (rc) return failed(rc, add ? "fused_add_rmsnorm_fp8_quant" : "rmsnorm_fp8_quant");
         return out.take();
     });
@@ -176,10 +184,11 @@ PyObject* silu(PyObject*, PyObject* const* args, Py_ssize_t n) {
         Ref out{pair(q, s)};
         if (!out.p) return nullptr;
         int rc;
-        Py_BEGIN_ALLOW_THREADS
-        rc = kbn_silu_mul_quant_fp8(x->data_ptr(), M, Nh, x->stride(0), q.data_ptr(), Nh, (float*)s.data_ptr(), s.stride(0),
-                                    s.stride(1), (float)PyFloat_AS_DOUBLE(args[2]), ue8m0, (void*)st);
-        Py_END_ALLOW_THREADS
+        {
+            NoGil no_gil;
+            rc = kbn_silu_mul_quant_fp8(x->data_ptr(), M, Nh, x->stride(0), q.data_ptr(), Nh, (float*)s.data_ptr(), s.stride(0),
+                                        s.stride(1), (float)PyFloat_AS_DOUBLE(args[2]), ue8m0, (void*)st);
+        }
         if (rc) return failed(rc, "silu_mul_quant_fp8");
         return out.take();
     });
@@ -249,11 +258,12 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
             const at::Tensor buf = bytes ? kept_workspace(args[8], dev, st, bytes) : at::Tensor();
             if (bytes && !buf.defined()) Py_RETURN_NONE;
             void* const wsp = bytes ? buf.data_ptr() : nullptr;
-            Py_BEGIN_ALLOW_THREADS
-            rc = kbn_fp8_gemm_bf16a(x->data_ptr(), x->stride(0), kQuantEps, w->data_ptr(), w->stride(0),
-                                    (const float*)ws->data_ptr(), ws->stride(0), o->data_ptr(), o->stride(0), M, N, K, wsp,
-                                    bytes, (void*)st);
-            Py_END_ALLOW_THREADS
+            {
+                NoGil no_gil;
+                rc = kbn_fp8_gemm_bf16a(x->data_ptr(), x->stride(0), kQuantEps, w->data_ptr(), w->stride(0),
+                                        (const float*)ws->data_ptr(), ws->stride(0), o->data_ptr(), o->stride(0), M, N, K, wsp,
+                                        bytes, (void*)st);
+            }
         } else {
             const at::Tensor *q = plain_tensor(qo), *s = plain_tensor(so);
             if (!q || !s || !is(*q, at::kFloat8_e4m3fn, dev, 2) || !is(*s, at::kFloat, dev, 2) || q->size(0) < M ||
@@ -263,12 +273,13 @@ PyObject* linear(PyObject*, PyObject* const* args, Py_ssize_t n) {
             const at::Tensor buf = bytes ? kept_workspace(args[8], dev, st, bytes) : at::Tensor();
             if (bytes && !buf.defined()) Py_RETURN_NONE;
             void* const wsp = bytes ? buf.data_ptr() : nullptr;
-            Py_BEGIN_ALLOW_THREADS
-            rc = kbn_fp8_linear_forward(x->data_ptr(), M, K, x->stride(0), q->data_ptr(), q->stride(0),
-                                        (float*)s->data_ptr(), s->stride(0), s->stride(1), kQuantEps, 1, w->data_ptr(),
-                                        w->stride(0), (const float*)ws->data_ptr(), ws->stride(0), o->data_ptr(),
-                                        o->stride(0), N, ue8m0, wsp, bytes, (void*)st);
-            Py_END_ALLOW_THREADS
+            {
+                NoGil no_gil;
+                rc = kbn_fp8_linear_forward(x->data_ptr(), M, K, x->stride(0), q->data_ptr(), q->stride(0),
+                                            (float*)s->data_ptr(), s->stride(0), s->stride(1), kQuantEps, 1, w->data_ptr(),
+                                            w->stride(0), (const float*)ws->data_ptr(), ws->stride(0), o->data_ptr(),
+                                            o->stride(0), N, ue8m0, wsp, bytes, (void*)st);
+            }
         }
         if (rc) return failed(rc, direct ? "fp8_gemm_bf16a" : "fp8_linear_forward");
         if (o->size(0) == M) {

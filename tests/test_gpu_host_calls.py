@@ -147,3 +147,16 @@ def test_a_flag_without_a_truth_value(gpu_device):
     with pytest.raises(ZeroDivisionError, match="no truth value"):
         SiluMulQuantFp8()(x, use_ue8m0=Bad())
     _same(SiluMulQuantFp8()(x, use_ue8m0=[]), SiluMulQuantFp8()(x, use_ue8m0=False))
+
+
+def test_an_exception_inside_the_step_is_left_to_python(gpu_device):
+    """Reading a tensor's address may throw in C++, and does so while the step
+    holds no GIL: the step takes it again and the Python path reports the error."""
+    x = torch.ones(61, 2048, device=gpu_device, dtype=BF16)
+    w = torch.ones(2048, device=gpu_device, dtype=BF16)
+    y = x.clone()
+    torch._C._set_throw_on_mutable_data_ptr(y)
+    assert _ops._host.norm(y, w, 1e-6, None) is None
+    with pytest.raises(RuntimeError, match="data pointer"):
+        RMSNormFP8Quant()(y, w)
+    _same(RMSNormFP8Quant()(x, w), RMSNormFP8Quant()(x.clone(), w))
