@@ -447,7 +447,6 @@ static void plan_dense_tile(Schedule& s, int64_t M, int64_t N, int64_t K, bool a
             n.splits = sp;
             n.kb_per_split = kbps;
             n.ws_bytes = sp > 1 ? (int64_t)sp * tiles * t.bm * t.bn * 4 : 0;
-            n.ws_start = std::max(s.ws_bytes, s.ws_start);
             s = n;
         }
     }
@@ -706,10 +705,7 @@ extern "C" int kbn_fp8_gemm_nt(const void* A, int64_t lda, const float* sA, int6
 
 extern "C" int64_t kbn_fp8_gemm_nt_workspace_bytes(int64_t M, int64_t N, int64_t K, int scale_ue8m0) {
     if (M <= 0 || N <= 0 || K <= 0 || K % kGroup != 0 || M > 0x7FFFFFFFLL || N > 0x7FFFFFFFLL) return 0;
-    // at least what the starting plan (128x128 or 256x256 tiles) would write,
-    // so what a caller holds for a shape does not hang on which tile is taken
-    const Schedule s = dense_schedule(M, N, K, scale_ue8m0, true);
-    return std::max(s.ws_bytes, s.ws_start);
+    return dense_schedule(M, N, K, scale_ue8m0, true).ws_bytes;
 }
 
 extern "C" int kbn_fp8_gemm_nt_ws(const void* A, int64_t lda, const float* sA, int64_t sA_stride_m,

@@ -1430,7 +1430,6 @@ struct Schedule {
     int64_t dp_tiles = 0;         // tiles [0, dp_tiles) data-parallel
     int splits = 1, kb_per_split = 0;  // the tail [dp_tiles, tiles)
     int64_t ws_bytes = 0;         // fp32 slabs of the tail
-    int64_t ws_start = 0;         // and those of the plan this one replaced (plan_dense_tile)
     bool fused = false;           // the split launch sums the slabs itself
     int fuse_a = 0;               // bf16 activations quantized by the GEMM: rows of four per wavefront (1, 2, 4)
     // 256-row tiles only: the last n192 columns run as 256x192 tiles in a

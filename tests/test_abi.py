@@ -117,22 +117,28 @@ def test_gemm_split_plan_choices():
     if torch.cuda.device_count() > 0 and torch.cuda.get_device_properties(0).multi_processor_count != 256:
         pytest.skip("the plan depends on the device's CU count; pinned for 256 CUs")
 
-    def splits(M, N, K, bm, bn):
-        tiles = -(-M // bm) * -(-N // bn)
-        return L.kbn_fp8_gemm_nt_workspace_bytes(M, N, K, 1) // (tiles % 256 * bm * bn * 4) or 1
+    def plan(M, N, K):
+        p = _plan(L, M, N, K)
+        # what a caller is asked for is what the plan writes
+        assert L.kbn_fp8_gemm_nt_workspace_bytes(M, N, K, 1) == p[8] == (
+            p[5] * (p[3] - p[4]) * p[0] * p[1] * 4 if p[5] > 1 else 0)
+        return int(p[0]), int(p[1]), int(p[5])
 
     # 12 K blocks: data-parallel (measured 10.3 us against 20.1 us split in two)
-    assert splits(128, 12288, 1536, 128, 128) == 1
-    assert splits(128, 4096, 1536, 128, 128) == 1
-    assert splits(64, 12288, 1536, 64, 128) == 1
-    assert splits(8, 12288, 1536, 64, 128) == 1
+    assert plan(128, 12288, 1536) == (128, 128, 1)
+    assert plan(128, 4096, 1536) == (128, 128, 1)
+    assert plan(64, 12288, 1536) == (64, 128, 1)
+    assert plan(8, 12288, 1536) == (64, 128, 1)
     # long K: split, and not deeper than the sweep's best
-    assert splits(128, 12288, 7168, 128, 128) == 2
-    assert splits(128, 7168, 18432, 128, 128) == 4
-    assert splits(8, 10240, 8192, 64, 128) == 3
-    assert splits(64, 8192, 28672, 64, 128) == 4
-    assert 6 <= splits(32, 2048, 7168, 64, 128) <= 8
-    assert splits(512, 4096, 7168, 256, 256) == 4
+    assert plan(128, 7168, 18432) == (128, 128, 4)
+    assert plan(8, 10240, 8192) == (64, 128, 3)
+    assert plan(64, 8192, 28672) == (64, 128, 4)
+    assert plan(32, 2048, 7168)[:2] == (64, 64) and 6 <= plan(32, 2048, 7168)[2] <= 8
+    # or smaller tiles over the whole of K: no slabs, and none asked for
+    assert plan(128, 12288, 7168) == (128, 64, 1)
+    assert plan(512, 4096, 7168) == (128, 64, 1)
+    assert plan(200, 8192, 8192) == (128, 64, 1)
+    assert plan(777, 4608, 7168) == (64, 256, 1)
 
 
 def test_gemm_ws_rejects_bad_shapes():
@@ -692,7 +698,7 @@ def test_dense_plans_above_64_rows_are_launchable():
         if splits > 1:
             slots = 256 * (2 if stages * ((bm + bn) * 128 + 2048) <= 80 * 1024 else 1)
             assert (n - dp) * splits <= slots and ws == splits * (n - dp) * bm * bn * 4 <= 64 << 20, (M, N, K, p)
-        assert L.kbn_fp8_gemm_nt_workspace_bytes(M, N, K, 1) >= ws
+        assert L.kbn_fp8_gemm_nt_workspace_bytes(M, N, K, 1) == ws
         assert np.array_equal(p, _plan(L, M, N, K))
 
 

@@ -75,6 +75,101 @@ def test_linear_same_as_python_path(gpu_device, monkeypatch, M):
     _same(*_both(monkeypatch, call))
 
 
+def _linear(gpu_device, M, N=2048, K=2048, seed=0):
+    from kb_nano_amd.fp8_linear import _block_requant
+    g = torch.Generator(device=gpu_device).manual_seed(seed + M)
+    w, ws = _block_requant(torch.randn(N, K, device=gpu_device, generator=g) * 0.02, True)
+    x = torch.randn(M, K, device=gpu_device, generator=g).to(BF16)
+    lin = Fp8Linear()
+    lin._ensure_buffers(M, K, N, gpu_device)
+    return lin, x, w, ws
+
+
+# weights whose plan splits K, by the row count: summed in the split launch, and by a launch of its own
+_SPLIT = {16: (2048, 2048), 100: (512, 7168)}
+
+
+def _native(lin, x, w, ws):
+    from kb_nano_amd.fp8_linear import is_e8m0_used
+    return _ops._host.linear(x, w, ws, lin._a_buf, lin._s_buf, lin._o_buf, lin._pf, is_e8m0_used(), _ops._WS_BUFS)
+
+
+@pytest.mark.parametrize("M", [16, 100])
+def test_linear_on_side_streams_and_threads(gpu_device, M):
+    """Each stream has its own split workspace; a side stream, and two threads
+    on streams of their own at once, give the default stream's bits."""
+    import threading
+    N, K = _SPLIT[M]
+    lin, x, w, ws = _linear(gpu_device, M, N, K)
+    assert (_ops.lib().kbn_fp8_gemm_nt_workspace_bytes(M, N, K, 1) if M > 64 else
+            _ops.lib().kbn_fp8_gemm_bf16a_workspace_bytes(M, N, K)) > 0
+    ref = lin(x, w, ws).clone()
+    torch.cuda.synchronize()
+    got, errors = {}, []
+
+    def work(name):
+        try:
+            mine = Fp8Linear()
+            mine._ensure_buffers(M, K, N, gpu_device)
+            stream = torch.cuda.Stream()
+            with torch.cuda.stream(stream):
+                first = mine(x, w, ws).clone()         # this stream's workspace is made by the Python path
+                assert (0, stream.cuda_stream) in _ops._WS_BUFS
+                for _ in range(20):
+                    out = mine(x, w, ws)
+                assert _native(mine, x, w, ws) is not None
+                got[name] = [first, out.clone()]
+            stream.synchronize()
+        except BaseException as e:                     # an assertion of a thread fails the test below
+            errors.append(e)
+    work("side stream")
+    threads = [threading.Thread(target=work, args=(i,)) for i in range(2)]
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    assert not errors, errors
+    assert len(got) == 3
+    for outs in got.values():
+        for out in outs:
+            assert torch.equal(out, ref)
+
+
+@pytest.mark.parametrize("M", [16, 100])
+def test_linear_with_a_kept_workspace_that_is_too_small(gpu_device, M):
+    lin, x, w, ws = _linear(gpu_device, M, *_SPLIT[M])
+    ref = lin(x, w, ws).clone()
+    key = (0, torch.cuda.current_stream().cuda_stream)
+    full = _ops._WS_BUFS[key]
+    _ops._WS_BUFS[key] = small = torch.empty(64, dtype=torch.uint8, device=gpu_device)
+    lin._o_buf.fill_(float("nan"))
+    assert _native(lin, x, w, ws) is None
+    assert torch.equal(lin(x, w, ws), ref)             # the Python path makes a larger one
+    assert _ops._WS_BUFS[key] is not small and _native(lin, x, w, ws) is not None
+    _ops._WS_BUFS[key] = full
+
+
+@pytest.mark.parametrize("M", [16, 100])
+def test_linear_refusals_are_the_python_path_s(gpu_device, M):
+    """What the entry points refuse, the step leaves to the Python path, which raises."""
+    lin, x, w, ws = _linear(gpu_device, M)
+    lin(x, w, ws)   # the split workspace of this stream exists afterwards
+    assert _native(lin, x, w, ws) is not None
+    flat = torch.zeros(M * 2048 + 8, device=gpu_device, dtype=BF16)
+    cases = {
+        "misaligned rows": (flat[1:1 + M * 2048].view(M, 2048), w, ws),
+        "row stride": (torch.zeros(M, 2049, device=gpu_device, dtype=BF16)[:, :2048], w, ws),
+        "too few scale rows": (x, w, ws[:8]),
+        "scales not along K": (x, w, ws.t().contiguous().t()),
+        "fp16 weight": (x, w.to(torch.float16), ws),
+    }
+    for name, args in cases.items():
+        assert _native(lin, *args) is None, name
+        with pytest.raises((RuntimeError, ValueError, TypeError)):
+            lin(*args)
+    assert torch.equal(lin(x, w, ws), lin(x.clone(), w, ws))
+
+
 def test_anything_but_the_plain_case_is_left_to_python(gpu_device):
     h = _ops._host
     x, w = torch.zeros(4, 256, device=gpu_device, dtype=BF16), torch.zeros(256, device=gpu_device, dtype=BF16)
