@@ -346,48 +346,58 @@ static void plan_mixed_192(Schedule& s, int64_t M, int64_t N) {
 // Modelled time of the dense UE8M0 tiles above 64 rows, in microseconds: what
 // decides is how a shape's tiles fill the CUs, so each tile is priced and the
 // cheapest taken.  A wave of w workgroups of kb K blocks takes
-//   kb (block + busy w / slots + fetch MB) + wave
-// with MB the distinct A and W rows of one K step over the wave, and the call
-// at least 2 us plus its bytes at `rate` TB/s.  Splitting K over s workgroups
-// a tile adds split + slab MB + s per.  Fitted to 234 shapes (M 72 to 4096
-// over 13 weights from 2048 x 2048 to 57344 x 8192 and 8192 x 28672, every
-// tile, 1 to 8 splits; 5-11% rms a tile).  Over those shapes the pick is 1.31x
-// faster than 128x128 (M <= 128) or 256x256 tiles throughout, and 3% from the
-// best tile measured.  Some of it, us: 200 x 2048 x 2048 20.2 -> 7.1
-// (64x64), 200 x 8192 x 8192 34.9 -> 22 (128x64), 777 x 4608 x 7168 44.8 ->
-// 33.5 (64x256), 1024 x 8192 x 8192 76 -> 56 (128x256, 8 wavefronts),
-// 1024 x 7168 x 18432 138 -> 121 (256x128).
+//   kb (block + busy w / slots + fetch MB [+ two]) + wave + out MB_out
+// with MB the distinct A and W rows of one K step over the wave, `two` where a
+// second workgroup shares a CU (the 64x64 tiles beyond one per CU: a block
+// then takes 0.5 us, not 0.25) and MB_out the bf16 tiles the wave leaves; the
+// call takes `start` more, and at least 2 us plus its bytes at `rate` TB/s.
+// Splitting K over s workgroups a tile adds split + slab MB + s per.
+//
+// Fitted to 33,600 timed plans of 2100 shapes: M 65 to 20000, N 64 to 60000
+// and K 512 to 30720, all spread over their logarithms, ragged N among them,
+// and 300 over the benchmark's weights; every tile, 1 to 8 splits, weights
+// and activations rotated past the caches.  On a third of the shapes left out
+// of the fit it is 7-11% rms off a tile's time, and the pick takes 0.71 of the
+// time of 128x128 (M <= 128) or 256x256 tiles throughout; 9 of those 700 are
+// slower by more than 2%, the worst 1.18 (125 x 10240 x 8192).  (A fit to 234
+// shapes of the 13 weights alone was up to 30% off other weights: 0.74, 55 of
+// the 2100 slower, the worst 1.5.)  Some of it, us: 200 x 2048 x 2048
+// 20.2 -> 7.1 (64x64), 200 x 8192 x 8192 34.9 -> 22 (128x64), 777 x 4608 x
+// 7168 44.8 -> 33.5 (64x256), 1024 x 8192 x 8192 76 -> 56 (128x256, 8
+// wavefronts), 1024 x 7168 x 18432 138 -> 121 (256x128).
 struct DenseTile {
     int bm, bn, stages, waves;
-    double block, busy, fetch, wave, start, split, slab, per, rate;
+    double block, busy, two, fetch, wave, start, split, slab, per, rate, out;
     // workgroups the chip holds at once: two per CU where two fit its LDS
     int64_t slots() const {
         return (int64_t)cu_count() * (stages * ((bm + bn) * kRowB + waves * 512) <= 80 * 1024 ? 2 : 1);
     }
 };
 constexpr DenseTile kDenseTiles[] = {
-    {64, 64, 4, 4, 0.113, 0.321, 0.008, 0.328, 3.768, 4.046, 0.040, 0.411, 3.578},
-    {128, 64, 4, 4, 0.242, 0.106, 0.007, 1.495, 2.075, 4.062, 0.141, 0.390, 4.248},
-    {64, 256, 3, 4, 0.342, 0.244, 0.071, 1.877, 1.755, 5.051, 0.000, 0.084, 4.257},
-    {128, 128, 4, 4, 0.415, 0.173, 0.026, 3.168, 1.273, 2.282, 0.471, 0.254, 4.883},
-    {128, 256, 3, 8, 0.479, 0.316, 0.068, 3.622, 0.389, 2.799, 0.237, 0.000, 4.700},
-    {256, 128, 3, 4, 0.578, 0.251, 0.000, 5.057, 0.171, 2.016, 0.409, 0.378, 4.876},
-    {192, 256, 2, 4, 0.967, 0.233, 0.084, 1.821, 0.000, 0.000, 0.308, 0.405, 6.036},
-    {256, 256, 2, 4, 1.094, 0.346, 0.060, 3.163, 0.000, 0.000, 0.312, 0.318, 3.954},
+    {64, 64, 4, 4, 0.232, 0.031, 0.158, 0.040, 0.000, 2.613, 1.758, 0.680, 0.157, 3.417, 0.308},
+    {128, 64, 4, 4, 0.280, 0.060, 0.000, 0.049, 0.946, 2.089, 2.156, 0.560, 0.144, 4.706, 0.230},
+    {64, 256, 3, 4, 0.507, 0.053, 0.000, 0.086, 0.000, 2.874, 3.584, 0.437, 0.086, 5.655, 0.240},
+    {128, 128, 4, 4, 0.534, 0.078, 0.000, 0.011, 0.269, 3.325, 2.427, 0.587, 0.092, 5.466, 0.307},
+    {128, 256, 3, 8, 0.701, 0.015, 0.000, 0.061, 2.255, 1.996, 2.577, 0.364, 0.101, 5.386, 0.140},
+    {256, 128, 3, 4, 0.678, 0.138, 0.000, 0.000, 2.705, 1.869, 3.281, 0.455, 0.038, 4.994, 0.135},
+    {192, 256, 2, 4, 1.130, 0.050, 0.000, 0.054, 2.271, 2.506, 5.017, 0.291, 0.000, 6.033, 0.096},
+    {256, 256, 2, 4, 1.193, 0.204, 0.000, 0.035, 2.484, 1.698, 6.882, 0.282, 0.108, 4.350, 0.135},
 };
 constexpr int kTile128 = 3, kTile256 = 7;   // the tiles of M <= 128 and M > 128 before the others are priced
 
 // Modelled time of `full` waves of whole-K tiles and then `rest` tiles (fewer
 // than a wave) in `splits` pieces of K.
 static double dense_cost(const DenseTile& t, int64_t M, int64_t N, int64_t K, double full, int64_t rest, int splits) {
-    const int64_t slots = t.slots();
+    const int64_t slots = t.slots(), cus = cu_count();
     const int64_t tm = (M + t.bm - 1) / t.bm, tn = (N + t.bn - 1) / t.bn, kbt = K / kGroup;
+    const double out_mb = 2.0 * (double)M * (double)N / (double)(tm * tn) / 1e6;   // one tile's outputs
     auto wave = [&](double w, int s) {   // one wave of w workgroups, s to a tile
         const double tiles = w / s, kb = (double)((kbt + s - 1) / s);
         const double cols = std::min<double>((double)tn, std::max(1.0, tiles / (double)tm));
         const double rows = std::min<double>((double)tm, std::max(1.0, tiles));
-        const double mb = (cols * t.bn + rows * t.bm) * kRowB * s / 1e6;
-        return kb * (t.block + t.busy * w / (double)slots + t.fetch * mb) + t.wave;
+        const double mb = (cols * t.bn + std::min<double>(rows * t.bm, (double)M)) * kRowB * s / 1e6;
+        return kb * (t.block + t.busy * w / (double)slots + (w > (double)cus ? t.two : 0.0) + t.fetch * mb) + t.wave +
+               (s > 1 ? 0.0 : t.out * out_mb * w);
     };
     double us = t.start + full * wave((double)slots, 1);
     if (rest > 0) us += wave((double)(rest * splits), splits);
@@ -402,16 +412,19 @@ static double dense_cost(const DenseTile& t, int64_t M, int64_t N, int64_t K, do
 }
 
 // Replaces s, the 128x128 or 256x256 plan, by the tile priced cheapest if that
-// saves at least 5%, or 15% for 256-column tiles up to 128 rows (less is within
-// the model's error: with 4% everywhere 65 x 36864 x 7168 took 128x256 tiles,
-// 66.5 us against 58.7, and 640 x 36864 x 7168 177.6 against 174.6).  The fit
-// holds no grids of a few workgroups, so they keep their plan (65 x 512 x 7168
-// in 16 workgroups of 128x256: 15.4 us against 12.4 of 128x128).  K of at most 12
+// saves at least 5%, or 20% for K of at most 4 blocks (where the outputs
+// decide and the prices are furthest off: 1435 x 5136 x 512, priced 18%
+// cheaper on 128x256 tiles, measured 18.8 us against 12.2).  Grids of a few workgroups
+// keep their plan (65 x 512 x 7168 in 16 workgroups of 128x256: 15.4 us
+// against 12.4 of 128x128).  K of at most 12
 // blocks keeps 128x128 for up to 128 rows, although 64x64 measured faster
 // there (3072 x 1536 at 128 rows 7.0 against 10.7 us): those plans, and that
 // a row's result does not depend on the row count under them, are held by
 // tests.
-constexpr int64_t kKeep128Kb = 12, kMinWorkgroups = 32;
+// Above 4096 rows 256x128 tiles have to save 20% as well: over many waves they
+// fetch more than their price, fitted to no fetch term, says (15387 x 1152 x
+// 2432 55.8 -> 59.1 us, 31462 x 1152 x 4352 145 -> 164).
+constexpr int64_t kKeep128Kb = 12, kMinWorkgroups = 32, kShortKb = 4, kManyRows = 4096;
 
 static void plan_dense_tile(Schedule& s, int64_t M, int64_t N, int64_t K, bool allow_split) {
     const int64_t kbt = K / kGroup;
@@ -426,7 +439,7 @@ static void plan_dense_tile(Schedule& s, int64_t M, int64_t N, int64_t K, bool a
     } else {
         best = dense_cost(old, M, N, K, (double)(s.tiles / cus), s.tiles % cus, s.splits);
     }
-    best *= 0.95;
+    best *= kbt <= kShortKb ? 0.80 : 0.95;
     for (const DenseTile& t : kDenseTiles) {
         if (&t == &old) continue;
         const int64_t slots = t.slots();
@@ -437,7 +450,7 @@ static void plan_dense_tile(Schedule& s, int64_t M, int64_t N, int64_t K, bool a
             if (pieces != sp) continue;
             const double us = sp > 1 ? dense_cost(t, M, N, K, 0, tiles, sp)
                                      : dense_cost(t, M, N, K, (double)(tiles / slots), tiles % slots, 1);
-            const double bias = M <= 128 && t.bn == 256 ? 0.95 / 0.85 : 1.0;
+            const double bias = M > kManyRows && t.bm == 256 && t.bn == 128 ? 0.95 / 0.80 : 1.0;
             if (us * bias >= best || tiles * sp < kMinWorkgroups) continue;
             best = us * bias;
             Schedule n;

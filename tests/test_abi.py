@@ -702,6 +702,25 @@ def test_dense_plans_above_64_rows_are_launchable():
         assert np.array_equal(p, _plan(L, M, N, K))
 
 
+@pytest.mark.parametrize("M,N,K,slow,us", [
+    (77, 1152, 7936, (64, 64, 1), (18.6, 12.3)), (68, 1152, 7168, (64, 64, 1), (17.4, 11.7)),
+    (70, 1664, 7808, (64, 64, 1), (18.5, 12.7)), (82, 1536, 7296, (64, 64, 1), (17.6, 13.3)),
+    (124, 1152, 6016, (64, 64, 1), (15.9, 12.7)), (104, 8832, 6528, (64, 64, 1), (30.6, 25.3)),
+    (70, 10240, 8192, (128, 64, 1), (27.9, 24.1)), (112, 10240, 8192, (128, 64, 1), (31.3, 27.4)),
+    (98, 35760, 3072, (128, 64, 1), (40.1, 35.2)), (101, 2816, 23552, (128, 64, 4), (27.0, 23.7)),
+    (120, 3952, 27904, (128, 64, 3), (43.2, 33.5)), (6682, 152, 28928, (256, 128, 4), (83.6, 71.6)),
+    (25000, 2944, 26880, (256, 128, 1), (1927, 1627)), (15387, 1152, 2432, (256, 128, 1), (59.1, 55.8))])
+def test_dense_plans_away_from_the_benchmark_s_weights(M, N, K, slow, us):
+    """Shapes on which prices fitted to the benchmark's weights alone (the last:
+    to all weights, but not above 4096 rows) took a tile that measured slower
+    than the 128x128 or 256x256 plan it replaced (`us`, both): two 64x64
+    workgroups on a CU, 128x64 tiles of long K or wide N, 256x128 tiles of many
+    waves or long K."""
+    from kb_nano_amd._lib import lib
+    p = _plan(lib(), M, N, K)
+    assert (p[0], p[1], p[5]) != slow, (p, us)
+
+
 def test_scales_are_pow2_predicate_and_cache():
     """The check that lets the MoE layers run the UE8M0 kernels under the
     FP32 contract: true only when every scale is a positive, finite, normal

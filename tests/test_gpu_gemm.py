@@ -906,10 +906,10 @@ def test_gemm_whole_line_store_paths(gpu_device, M, N, K, tile):
     assert np.array_equal(bf16_bits(D1), bf16_bits(D[:M - 1])), "rows depend on the row count"
 
 
-@pytest.mark.parametrize("M,N,K,tile", [(452, 200, 1024, (64, 64, 1)), (66, 200, 7168, (64, 64, 4)),
-                                        (194, 8200, 1024, (64, 256, 1)), (899, 200, 8192, (64, 256, 8)),
+@pytest.mark.parametrize("M,N,K,tile", [(452, 200, 1024, (64, 64, 1)), (66, 200, 7168, (64, 64, 8)),
+                                        (194, 8200, 1024, (64, 256, 1)), (144, 2752, 11648, (64, 256, 7)),
                                         (200, 8192, 8192, (128, 64, 1)), (65, 3000, 8192, (128, 64, 5)),
-                                        (515, 7176, 1024, (128, 256, 1)), (129, 328, 4096, (128, 256, 8)),
+                                        (515, 7176, 1024, (128, 256, 1)), (134, 5552, 7808, (128, 256, 5)),
                                         (905, 8200, 1024, (192, 256, 1)), (2459, 3080, 1664, (256, 128, 1))])
 def test_gemm_dense_tile_choice(gpu_device, M, N, K, tile):
     """Each tile the dense planner picks above 64 rows besides 128x128 and
