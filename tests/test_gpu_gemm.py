@@ -51,10 +51,14 @@ def test_gemm_matches_oracle(gpu_device, M, N, K, ue8m0):
 def test_gemm_k_blocks_against_stages(gpu_device, M, ue8m0):
     """Every number of K blocks from one to nine, i.e. fewer than a tile's LDS
     stages (two to four), whole rounds of them and every remainder, on 64-,
-    128- and 256-row tiles; 23 blocks may be split over K."""
+    128- and 256-row tiles (UE8M0; up to seven blocks, more may take smaller
+    tiles and split K); 23 blocks are split over K."""
     N = 320
     for KB in (1, 2, 3, 4, 5, 6, 7, 8, 9, 23):
         K = 128 * KB
+        if KB <= 7 or KB == 23:
+            p = _plan(M, N, K)
+            assert p[5] > 1 if KB == 23 else (p[0], p[5]) == ({20: 64, 100: 128, 300: 256}[M], 1), p
         qa, sa, qw, sw = quantized_gemm_inputs(M, N, K, seed=M + KB)
         if not ue8m0:
             sw = (sw * np.float32(1.37)).astype(np.float32)
@@ -685,16 +689,21 @@ def test_gemm_fused_splitk_forked_capture(gpu_device):
         assert np.array_equal(bf16_bits(extra), eager[1]), f"eager call between replays {rep}"
 
 
-@pytest.mark.parametrize("M,N,K", [(100, 2304, 4096), (1, 7168, 18432), (8, 8192, 8192), (64, 2048, 2048),
-                                   (77, 200, 1152), (300, 1024, 2048), (512, 768, 8704)])
-def test_gemm_packed_row_scales_equal_block_scales(gpu_device, M, N, K):
+@pytest.mark.parametrize("M,N,K,tile", [(100, 2304, 4096, (64, 64, 3)), (1, 7168, 18432, (64, 128, 4)),
+                                        (8, 8192, 8192, (64, 128, 4)), (64, 2048, 2048, (64, 64, 4)),
+                                        (77, 200, 1152, (128, 128, 1)), (70, 80, 1664, (128, 128, 3)),
+                                        (300, 1024, 2048, (64, 64, 1)), (512, 768, 8704, (128, 64, 4))])
+def test_gemm_packed_row_scales_equal_block_scales(gpu_device, M, N, K, tile):
     """DeepGEMM's packed per-row UE8M0 weight scales (int32 [N, ceil(K/512)],
     MN-major; the reference's own fp8_linear scenarios pass this layout,
     bench/kernels/benchmark_scenarios/small/shape_registry.yaml:18719-18737):
     with the block scales' exponents repeated on every row of a block, the
     output is the fp32-block-scale GEMM's bit for bit (data-parallel, split
-    tails summed in the split launch and by the reduction, 128x128 and
-    256x256 tiles, K not a multiple of 512), every output written."""
+    tails summed in the split launch and by the reduction, on tiles of up to
+    128 rows as planned, K not a multiple of 512), every output written.
+    test_gemm_dense_tile_choice has the larger tiles."""
+    p = _plan(M, N, K)
+    assert (p[0], p[1], p[5]) == tile, p
     from kb_nano_amd import _ops
     from tests._util import assert_all_written
     qa, sa, qw, sw = quantized_gemm_inputs(M, N, K, seed=M + 2 * N + K)
@@ -906,20 +915,28 @@ def test_gemm_whole_line_store_paths(gpu_device, M, N, K, tile):
     assert np.array_equal(bf16_bits(D1), bf16_bits(D[:M - 1])), "rows depend on the row count"
 
 
-@pytest.mark.parametrize("M,N,K,tile", [(452, 200, 1024, (64, 64, 1)), (66, 200, 7168, (64, 64, 8)),
-                                        (194, 8200, 1024, (64, 256, 1)), (144, 2752, 11648, (64, 256, 7)),
-                                        (200, 8192, 8192, (128, 64, 1)), (65, 3000, 8192, (128, 64, 5)),
-                                        (515, 7176, 1024, (128, 256, 1)), (134, 5552, 7808, (128, 256, 5)),
-                                        (905, 8200, 1024, (192, 256, 1)), (2459, 3080, 1664, (256, 128, 1))])
+@pytest.mark.parametrize("M,N,K,tile", [
+    (452, 200, 1024, (64, 64, 1)), (66, 200, 7168, (64, 64, 8)),
+    (194, 8200, 1024, (64, 256, 1)), (144, 2752, 11648, (64, 256, 7)),
+    (200, 8192, 8192, (128, 64, 1)), (65, 3000, 8192, (128, 64, 5)),
+    (515, 7176, 1024, (128, 256, 1)), (134, 5552, 7808, (128, 256, 5)),
+    (905, 8200, 1024, (192, 256, 1)), (1056, 7528, 640, (192, 256, 1)), (137, 10984, 8320, (192, 256, 5)),
+    (2459, 3080, 1664, (256, 128, 1)), (135, 3688, 12160, (256, 128, 8)),
+    # 256x256: eight wavefronts (K up to 2048) whole and split, four whole, split and with a split tail
+    (182, 72, 640, (256, 256, 1)), (151, 64, 1664, (256, 256, 3)),
+    (971, 10992, 2176, (256, 256, 1)), (133, 112, 2688, (256, 256, 5)), (3332, 4664, 2176, (256, 256, 3)),
+    (898, 8256, 8320, (256, 256, 1))])   # the last columns on 256x192 tiles
 def test_gemm_dense_tile_choice(gpu_device, M, N, K, tile):
-    """Each tile the dense planner picks above 64 rows besides 128x128 and
-    256x256, whole and split over K, at ragged M and N: the NaN-prefilled
-    output is fully written and matches the oracle in every 64x64 block, and
-    packed per-row weight scales give the same bits."""
+    """Each tile the dense planner picks above 64 rows besides 128x128, whole
+    and split over K, at ragged M and N and, for the tiles of two LDS stages,
+    odd numbers of K blocks: the NaN-prefilled output is fully written and
+    matches the oracle in every 64x64 block, and packed per-row weight scales
+    give the same bits."""
     from kb_nano_amd import _ops
     from tests._util import assert_all_written, tile_cover
     p = _plan(M, N, K)
     assert (p[0], p[1], p[5]) == tile, p
+    assert (p[3] != -(-M // p[0]) * -(-N // p[1])) == (K == 8320 and M == 898), f"256x192 tiles: {p}"
     qa, sa, qw, sw = quantized_gemm_inputs(M, N, K, seed=M + 5 * N + K)
     D = _gemm_gpu(qa, sa, qw, sw, gpu_device)
     assert_all_written(D, f"{M}x{N}x{K}")
