@@ -21,6 +21,15 @@ namespace kbn {
 #endif
 constexpr int64_t kPadZeroMaxK = KBN_PAD_ZERO_MAX_K;
 
+// Contiguous-layout grouped GEMMs with UE8M0 scales take four wavefronts a
+// tile from this K and this many layout rows an expert on: an 8-wavefront tile
+// reads a third more from LDS per MFMA, which shows once the K loop is all there
+// is.  gate_up 4096 x 7168 of 256 experts, us, four against eight, two boxes:
+// 4096 tokens (255 rows an expert) 1729 / 1779 and 1687 / 1732, 1500 (174) 1279 /
+// 1296 and 1236 / 1252, 515 (143) 1250 / 1253 and 1207 / 1202, 128 (131) 1184 /
+// 1170; K = 4096 (128 experts, 4096 tokens) 598 / 560.
+constexpr int64_t kGroupedFourK = 6144, kGroupedFourRows = 160;
+
 // Only tails whose split workgroups fit in one wave are split (more waves
 // never measured faster, and the allocation-free entry point's scratch is
 // sized for one wave).  Cost model in microseconds, fitted to sweeps of the
@@ -910,12 +919,17 @@ extern "C" int kbn_fp8_grouped_gemm_nt_contiguous(const void* A, int64_t lda, co
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     // grouped: data-parallel, one workgroup per 128-row block x N tile, of
     // eight wavefronts: two per SIMD cover each other's waits, and the FP32
-    // contract's rescale is half as long per wavefront.  Experts layer, us,
-    // four -> eight (both GEMMs): 128 experts x 4096 x 1536, 515 tokens, scales
-    // as given 519 -> 484, 4096 tokens 1357 -> 1271; 256 x 7168 x 2048, 4096
-    // tokens 3253 -> 3129 as given, 2938 -> 2937 with powers of two.
+    // contract's rescale is half as long per wavefront.  us, four -> eight,
+    // one box, in turn (4096 tokens): 256 experts, gate_up 4096 x 7168 scales
+    // as given 1986 -> 1873, down 7168 x 2048 951 -> 946 (powers of two), 1119
+    // -> 1016 (as given); 128 experts, gate_up 3072 x 4096 598 -> 560, 758 ->
+    // 642, down 4096 x 1536 422 -> 393, 500 -> 432; 128 to 1500 tokens 1-14%
+    // faster.  kGroupedFourK: the one regime where four were faster.
     Schedule sc;
-    if (scale_ue8m0) return launch_gemm<128, 256, 3, true, true, 8>(a, sc, st, what);
+    if (scale_ue8m0) {
+        if (K >= kGroupedFourK && M_sum >= kGroupedFourRows * E) return launch_gemm<128, 256, 3, true, true, 4>(a, sc, st, what);
+        return launch_gemm<128, 256, 3, true, true, 8>(a, sc, st, what);
+    }
     return launch_gemm<128, 256, 3, false, true, 8>(a, sc, st, what);
 }
 

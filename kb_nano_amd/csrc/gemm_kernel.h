@@ -662,24 +662,32 @@ gemm_bs_kernel(const GemmArgs a) {
     auto a_off = [&](int i) -> int { if constexpr (kKeepOff || kGrouped) return va[i]; else return a_voff(i); };
     auto w_off = [&](int i) -> int { if constexpr (kKeepOff) return vw[i]; else return w_voff(i); };
     int s_fetch = 0;   // the block to fetch next (0, with A and W unreadable, past the last)
-    // Load unit u (0 <= u < kUnits) of the block to fetch next, into stage S:
-    // the scale vectors, then the A rows, then the W rows.
+    // Load unit u (0 <= u < kUnits) of the block to fetch next, into stage S
+    // (a constant, or an int in the rolled loop): the scale vectors, then the
+    // A rows, then the W rows.
     auto issue_unit = [&](auto S_, auto u_) {
-        constexpr int S = decltype(S_)::value, u = decltype(u_)::value;
+        constexpr int u = decltype(u_)::value;
+        constexpr bool kConst = !std::is_same_v<decltype(S_), int>;
+        constexpr int S = [] { if constexpr (kConst) return (int)decltype(S_)::value; else return 0; }();
+        const int rt = kConst ? 0 : (int)S_;
         if constexpr (!kFuseA && u == 0) {
-            dma_b32<kOffS + S * (kSA + kSW)>(dSA, lds_s, sa_off0, s_fetch * sa_kstep);
+            dma_b32<kOffS + S * (kSA + kSW)>(dSA, lds_s + rt * (kSA + kSW), sa_off0, s_fetch * sa_kstep);
         } else if constexpr (u == kScaleDma - 1) {
-            dma_b32<kOffS + S * (kSA + kSW) + kSA>(dSW, lds_s, sw_off0,
+            dma_b32<kOffS + S * (kSA + kSW) + kSA>(dSW, lds_s + rt * (kSA + kSW), sw_off0,
                                                    kRowW ? ((kb0 + s_fetch) >> 2) * sw_kstep : s_fetch * sw_kstep);
         } else if constexpr (u < kScaleDma + kAUnits) {
             constexpr int i = (u - kScaleDma) * (kPairA ? 2 : 1);
             const int soff = s_fetch * (kFuseA ? 2 * kRowB : kRowB);
-            if constexpr (kPairA) dma_b128_pair<S * kA + i * 1024, false>(dA, lds_a, a_off(i), a_off(i + 1), soff);
-            else dma_b128<S * kA + i * 1024, false>(dA, lds_a, a_off(i), soff);
+            if constexpr (kPairA)
+                dma_b128_pair<S * kA + i * 1024, false>(dA, lds_a + rt * kA, a_off(i), a_off(i + 1), soff);
+            else
+                dma_b128<S * kA + i * 1024, false>(dA, lds_a + rt * kA, a_off(i), soff);
         } else {
             constexpr int i = (u - kScaleDma - kAUnits) * (kPairW ? 2 : 1), off = kOffW + S * kB + i * 1024;
-            if constexpr (kPairW) dma_b128_pair<off, kWeightNt>(dW, lds_w, w_off(i), w_off(i + 1), s_fetch * kRowB);
-            else dma_b128<off, kWeightNt>(dW, lds_w, w_off(i), s_fetch * kRowB);
+            if constexpr (kPairW)
+                dma_b128_pair<off, kWeightNt>(dW, lds_w + rt * kB, w_off(i), w_off(i + 1), s_fetch * kRowB);
+            else
+                dma_b128<off, kWeightNt>(dW, lds_w + rt * kB, w_off(i), s_fetch * kRowB);
         }
     };
     // Past the last block the descriptors end at 0, so the A and W loads write
@@ -997,9 +1005,12 @@ gemm_bs_kernel(const GemmArgs a) {
     // left to fetch.
     auto block = [&](auto S_, auto fetch_, int kb) {
         constexpr bool kFetch = decltype(fetch_)::value;
-        constexpr int S = decltype(S_)::value, next = (S + 1) % kStages;
+        const int S = S_, next = S + 1 < kStages ? S + 1 : 0;
         // blocks' loads issued after those of block kb+1
-        constexpr int kAhead = kFetch ? kStages - 2 : std::max(kStages - 2 - S, 0);
+        constexpr int kAhead = [] {
+            if constexpr (kFetch) return kStages - 2;
+            else return std::max(kStages - 2 - (int)decltype(S_)::value, 0);
+        }();
         rescale_all();
         // ---- sub-step 0: K half 0 of block kb; read K half 1
 #pragma unroll
@@ -1074,12 +1085,20 @@ gemm_bs_kernel(const GemmArgs a) {
     // computed).  us a call, stage computed -> unrolled: 8 x 10240 x 8192
     // 19.0 -> 17.4, 64 x 2048 x 2048 9.3 -> 8.9, 4096 x 36864 x 7168 836 ->
     // 805.
-    int kb = 0;
-    for (; kb + kStages <= KB; kb += kStages)
-        static_for<kStages>([&](auto S_) { block(S_, std::true_type{}, kb + decltype(S_)::value); });
-    static_for<kStages - 1>([&](auto S_) {
-        if (kb + decltype(S_)::value < KB) block(S_, std::false_type{}, kb + decltype(S_)::value);
-    });
+    // Grouped tiles of four wavefronts keep the stage a variable: unrolled, the
+    // compiler moves their accumulators between register files (gate_up of 256
+    // experts at 4096 tokens 1729 -> 2022 us; kGroupedFourK says what they are
+    // for).
+    if constexpr (!(kGrouped && kWaves == 4)) {
+        int kb = 0;
+        for (; kb + kStages <= KB; kb += kStages)
+            static_for<kStages>([&](auto S_) { block(S_, std::true_type{}, kb + decltype(S_)::value); });
+        static_for<kStages - 1>([&](auto S_) {
+            if (kb + decltype(S_)::value < KB) block(S_, std::false_type{}, kb + decltype(S_)::value);
+        });
+    } else {
+        for (int kb = 0, st = 0; kb < KB; ++kb, st = st + 1 < kStages ? st + 1 : 0) block(st, std::true_type{}, kb);
+    }
     // the trailing (out-of-range) loads still target this workgroup's LDS
     wait_dma();
     if constexpr (!kUe8m0) {
@@ -1489,7 +1508,7 @@ static int launch_gemm(GemmArgs a, const Schedule& sc, hipStream_t st, const cha
             <<<dim3((unsigned)grid), dim3(64 * kWaves), 0, st>>>(a);
         KBN_CHECK_LAUNCH(what);
     }
-    if (dp < tiles) {
+    if constexpr (!kGrouped) if (dp < tiles) {
         // the plan must be for this tile shape, and its slabs must fit the workspace
         KBN_CHECK_ARG(sc.bm == BM && sc.bn == BN && sc.tiles == tiles && sc.fuse_a == kFuseA,
                       "%s: split plan does not match the %dx%d tiles", what, BM, BN);
@@ -1511,7 +1530,7 @@ static int launch_gemm(GemmArgs a, const Schedule& sc, hipStream_t st, const cha
         // less).  More rows: that sum would run on one workgroup per tile at
         // the end of the launch, so the separate kernel spreads it instead.
         a.flags = (BM <= 64 && sc.fused) ? splitk_flags_for(st, tiles - dp) : nullptr;
-        gemm_bs_kernel<BM, BN, kStages, kUe8m0, kGrouped && false, true, kWaves, false, kFuseA, kRowW>
+        gemm_bs_kernel<BM, BN, kStages, kUe8m0, false, true, kWaves, false, kFuseA, kRowW>
             <<<dim3((unsigned)blocks), dim3(64 * kWaves), 0, st>>>(a);
         KBN_CHECK_LAUNCH(what);
         if (!a.flags) {

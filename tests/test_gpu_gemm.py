@@ -320,6 +320,33 @@ def test_grouped_gemm_matches_oracle(gpu_device, ue8m0):
         assert torch.equal(C2, C)
 
 
+@pytest.mark.parametrize("K", [6144, 6272, 6400])
+def test_grouped_gemm_four_wavefronts(gpu_device, K):
+    """UE8M0 grouped GEMMs of at least 6144 K and 160 layout rows an expert run
+    four wavefronts a tile: every remainder of K blocks against its three
+    stages, N not a multiple of the tile, padding unwritten, close to the
+    oracle, and the bits of the eight-wavefront tiles (taken with more, unused,
+    experts)."""
+    from kb_nano_amd import _ops
+    E, N, dev = 3, 328, gpu_device
+    ids, qa, sa, qb, sb, M_sum = _grouped_case(E, N, K, M_tok=300, topk=2, seed=K, dev=dev)
+    assert 160 * E <= M_sum < 160 * (E + 4)
+    A, sA, idt = to_fp8(qa, dev), torch.from_numpy(sa).to(dev), torch.from_numpy(ids).to(dev)
+    outs = []
+    for extra in (0, 4):
+        B = to_fp8(np.concatenate([qb, qb[:1].repeat(extra, 0)]), dev)
+        sB = torch.from_numpy(np.concatenate([sb, sb[:1].repeat(extra, 0)])).to(dev)
+        C = torch.full((M_sum, N), 7.0, dtype=torch.bfloat16, device=dev)
+        _ops.m_grouped_gemm_nt_contiguous(A, sA, B, sB, C, idt, disable_ue8m0_cast=False)
+        outs.append(C)
+    torch.cuda.synchronize()
+    valid = ids >= 0
+    ref = oracle.grouped_gemm_nt_sample(qa, sa, qb, sb, ids)
+    assert_gemm_close(outs[0][torch.from_numpy(valid).to(dev)], ref[valid], f"four wavefronts, K={K}")
+    assert torch.all(outs[0][torch.from_numpy(~valid).to(dev)] == 7.0)
+    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+
+
 def test_grouped_gemm_free_function_colmajor_scales(gpu_device):
     """moe_grouped_gemm.py:71-83 path (disable_ue8m0_cast=True) with the
     column-major A scales SiluMulQuantFp8 produces."""
