@@ -791,18 +791,21 @@ extern "C" int64_t kbn_fp8_gemm_bf16a_workspace_bytes(int64_t M, int64_t N, int6
 }
 
 // Whether the bf16-activation GEMM is expected to beat quant + GEMM (the
-// separate quant launch costs 3-5 us per call on MI355X).  Up to 32 rows the
-// in-kernel quant of the 16 or 32 loaded rows costs each workgroup well under
-// that (measured on every Llama-70B decode shape and 2048/7168 x 2048: 0.5-4.7
-// us faster, gate_up at 32 rows even).  With 64 rows (16 per wavefront) it
-// costs about 0.1-0.3 us per K block, so it is taken only when the plan
-// splits K into workgroups of at most 16 blocks within one wave of tiles
-// (2048 x 2048, o); long K per workgroup (qkv 22, down 56 blocks), more
-// tiles than CUs (gate_up: its 102 KB stage set drops to one workgroup per
-// CU) and unsplit plans stay with quant + GEMM.  On the 64x64 tiles of narrow
-// weights the fp8 GEMM gains more than the in-kernel quant, so 64 rows take
-// it only for K <= 4096 (4096 x 7168: 17.5 us, against 11.3 us of GEMM plus
-// the 3-5 us quant launch; 2048 x 2048: 9.8 us against 7.4 us plus the quant).
+// quant is 2-3 us of GPU time more, and a launch).  Up to 32 rows the in-kernel
+// quant of the 16 or 32 loaded rows costs each workgroup less than that.  With
+// 64 rows (16 per wavefront) it costs about 0.1-0.3 us per K block, so it is
+// taken only when the plan splits K into workgroups of at most 16 blocks
+// within one wave of tiles (2048 x 2048, o); long K per workgroup (qkv 22,
+// down 56 blocks), more tiles than CUs and unsplit plans stay with quant +
+// GEMM, and so do the 64x64 tiles of narrow weights beyond K = 4096.
+// Both paths timed over 17 weights at 17 to 64 rows (graphs, weights rotated
+// past the caches; us, in-kernel quant / quant + GEMM): 32 rows of 2048 x 2048
+// 8.3 / 9.6, 8192 x 8192 17.6 / 19.7, 10240 x 8192 20.3 / 22.0; 64 rows of
+// 2048 x 2048 9.7 / 10.3, 8192 x 8192 21.3 / 22.6, and not taken 7168 x 2048
+// 15.1 / 12.6, 4096 x 7168 16.2 / 15.8, 10240 x 8192 25.5 / 24.8.  The rule
+// took the slower one at 20 of 119, by 1% or less but for 36864 x 7168 (32
+// rows 65.4 / 63.1, 33-64 rows 58.4-64.6 / 63.3-69.4), 7168 x 16384 (33-64 rows
+// 3-5%) and 8192 x 28672 (33 rows 2%).
 extern "C" int kbn_fp8_gemm_bf16a_preferred(int64_t M, int64_t N, int64_t K) {
     if (M <= 0 || M > 64 || N <= 0 || K <= 0 || K % kGroup != 0 || N > 0x7FFFFFFFLL) return 0;
     if (M <= 32) return 1;
