@@ -1323,7 +1323,7 @@ gemm_bs_kernel(const GemmArgs a) {
                 int roff;
                 if constexpr (kSorted) {
                     // the output row (routed pair) of wavefront row rl, held by
-                    // lane rl % 32 for fragment rl / 32 (rl / 32 is it / 8)
+                    // lane rl % 32 for fragment rl / 32 (the same for all lanes: kRowsPer divides 32)
                     const int orow = __shfl(out_row[(it * kRowsPer) / 32], rl & 31);
                     roff = orow >= 0 ? orow * (int)a.ldd * 2 : kOob;
                 } else if constexpr (kGrouped) {
