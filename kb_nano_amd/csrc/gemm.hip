@@ -21,14 +21,28 @@ namespace kbn {
 #endif
 constexpr int64_t kPadZeroMaxK = KBN_PAD_ZERO_MAX_K;
 
-// Contiguous-layout grouped GEMMs with UE8M0 scales take four wavefronts a
-// tile from this K and this many layout rows an expert on: an 8-wavefront tile
-// reads a third more from LDS per MFMA, which shows once the K loop is all there
-// is.  gate_up 4096 x 7168 of 256 experts, us, four against eight, two boxes:
-// 4096 tokens (255 rows an expert) 1729 / 1779 and 1687 / 1732, 1500 (174) 1279 /
-// 1296 and 1236 / 1252, 515 (143) 1250 / 1253 and 1207 / 1202, 128 (131) 1184 /
-// 1170; K = 4096 (128 experts, 4096 tokens) 598 / 560.
-constexpr int64_t kGroupedFourK = 6144, kGroupedFourRows = 160;
+// Contiguous-layout grouped GEMMs run eight wavefronts a tile, except where four
+// (with the K loop not unrolled) measured faster: long K, where the eight's
+// extra third of LDS reads per MFMA shows, and row-major activation scales,
+// which each wavefront gathers a cache line a row.  us, four / eight, in turn on
+// one box at a time; 256 experts gate_up 4096 x 7168, 128 experts 3072 x 4096,
+// tokens; "p" scales that are powers of two, "g" as given:
+//  - UE8M0, column-major, K = 7168: 4096 tokens (255 layout rows an expert)
+//    1729 / 1779, 1500 (174) 1279 / 1296, 515 (143) 1250 / 1253, 128 1184 /
+//    1170; K = 4096 (4096 tokens) 598 / 560.  Under the FP32 contract eight are
+//    4-6% faster with "g" and 1-4% slower with "p", which the host cannot tell.
+//  - row-major, K = 7168: 515 tokens 1354 / 1416 (UE8M0), 1357 / 1418 (p), 1362 /
+//    1413 (g); 1500 1376 / 1457 (p), 1382 / 1449 (g); 4096 1890 / 2023 (p), 2023 /
+//    2044 (g).  With SiLU*Mul 1379 / 1422 (p, 515), 2006 / 2081 (UE8M0, 4096).
+//  - row-major, K = 4096: 515 tokens (159 rows) 301 / 313 (p), 316 / 323 (UE8M0);
+//    1500 (221) 310 / 326 (p), 347 / 346 (g); 4096 (383) 631 / 658 (UE8M0), 639 /
+//    649 (p), but 748 / 675 (g).  With SiLU*Mul 644 / 669 (UE8M0, 4096), 755 /
+//    699 (g).  K up to 2048: eight, 2-12% faster.
+constexpr int64_t kGroupedFourK = 6144, kGroupedFourRows = 160, kGroupedFourRowMajorK = 4096, kGroupedFewRows = 300;
+static bool grouped_four(bool row_major, bool ue8m0, bool glu, int64_t M_sum, int64_t K, int64_t E) {
+    if (K >= kGroupedFourK) return row_major || (ue8m0 && !glu && M_sum >= kGroupedFourRows * E);
+    return K >= kGroupedFourRowMajorK && row_major && (ue8m0 || (!glu && M_sum < kGroupedFewRows * E));
+}
 
 // Only tails whose split workgroups fit in one wave are split (more waves
 // never measured faster, and the allocation-free entry point's scratch is
@@ -927,13 +941,14 @@ extern "C" int kbn_fp8_grouped_gemm_nt_contiguous(const void* A, int64_t lda, co
     // as given 1986 -> 1873, down 7168 x 2048 951 -> 946 (powers of two), 1119
     // -> 1016 (as given); 128 experts, gate_up 3072 x 4096 598 -> 560, 758 ->
     // 642, down 4096 x 1536 422 -> 393, 500 -> 432; 128 to 1500 tokens 1-14%
-    // faster.  kGroupedFourK: the one regime where four were faster.
+    // faster.  Four where grouped_four says so.
     Schedule sc;
-    if (scale_ue8m0) {
-        if (K >= kGroupedFourK && M_sum >= kGroupedFourRows * E) return launch_gemm<128, 256, 3, true, true, 4>(a, sc, st, what);
-        return launch_gemm<128, 256, 3, true, true, 8>(a, sc, st, what);
-    }
-    return launch_gemm<128, 256, 3, false, true, 8>(a, sc, st, what);
+    const bool four = grouped_four(sA_stride_m > 1 && sA_stride_k == 1, scale_ue8m0, false, M_sum, K, E);
+    if (scale_ue8m0)
+        return four ? launch_gemm<128, 256, 3, true, true, 4>(a, sc, st, what)
+                    : launch_gemm<128, 256, 3, true, true, 8>(a, sc, st, what);
+    return four ? launch_gemm<128, 256, 3, false, true, 4>(a, sc, st, what)
+                : launch_gemm<128, 256, 3, false, true, 8>(a, sc, st, what);
 }
 
 extern "C" int kbn_fp8_grouped_gemm_silu_quant(const void* A, int64_t lda, const float* sA, int64_t sA_stride_m,
@@ -979,8 +994,12 @@ extern "C" int kbn_fp8_grouped_gemm_silu_quant(const void* A, int64_t lda, const
     if (!a.silu_lut) return 1;
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
     Schedule sc;
-    if (scale_ue8m0) return launch_gemm<128, 256, 3, true, true, 8, 0, false, true>(a, sc, st, what);
-    return launch_gemm<128, 256, 3, false, true, 8, 0, false, true>(a, sc, st, what);
+    const bool four = grouped_four(sA_stride_m > 1 && sA_stride_k == 1, scale_ue8m0, true, M_sum, K, E);
+    if (scale_ue8m0)
+        return four ? launch_gemm<128, 256, 3, true, true, 4, 0, false, true>(a, sc, st, what)
+                    : launch_gemm<128, 256, 3, true, true, 8, 0, false, true>(a, sc, st, what);
+    return four ? launch_gemm<128, 256, 3, false, true, 4, 0, false, true>(a, sc, st, what)
+                : launch_gemm<128, 256, 3, false, true, 8, 0, false, true>(a, sc, st, what);
 }
 
 extern "C" int64_t kbn_fp8_fused_moe_gemm_workspace_bytes(int64_t EM, int64_t K) {

@@ -1087,7 +1087,7 @@ gemm_bs_kernel(const GemmArgs a) {
     // 805.
     // Grouped tiles of four wavefronts keep the stage a variable: unrolled, the
     // compiler moves their accumulators between register files (gate_up of 256
-    // experts at 4096 tokens 1729 -> 2022 us; kGroupedFourK says what they are
+    // experts at 4096 tokens 1729 -> 2022 us; grouped_four says what they are
     // for).
     if constexpr (!(kGrouped && kWaves == 4)) {
         int kb = 0;

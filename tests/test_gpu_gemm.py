@@ -320,31 +320,46 @@ def test_grouped_gemm_matches_oracle(gpu_device, ue8m0):
         assert torch.equal(C2, C)
 
 
-@pytest.mark.parametrize("K", [6144, 6272, 6400])
-def test_grouped_gemm_four_wavefronts(gpu_device, K):
-    """UE8M0 grouped GEMMs of at least 6144 K and 160 layout rows an expert run
-    four wavefronts a tile: every remainder of K blocks against its three
-    stages, N not a multiple of the tile, padding unwritten, close to the
-    oracle, and the bits of the eight-wavefront tiles (taken with more, unused,
-    experts)."""
+@pytest.mark.parametrize("ue8m0", [True, False])
+@pytest.mark.parametrize("K", [2048, 4096, 6144, 6272, 6400])
+def test_grouped_gemm_four_and_eight_wavefronts(gpu_device, K, ue8m0):
+    """Grouped GEMMs of long K run four wavefronts a tile for row-major
+    activation scales, and from K = 6144 under UE8M0 also for column-major ones
+    with at least 160 layout rows an expert; eight otherwise.  Every remainder
+    of K blocks against the tile's three stages, N not a multiple of the tile:
+    close to the oracle, padding unwritten, and the same bits from both scale
+    layouts and with more, unused, experts (fewer rows an expert).  The same
+    for the GEMM with SiLU*Mul + quant in its epilogue."""
     from kb_nano_amd import _ops
+    from kb_nano_amd.fp8_linear import _alloc_colmajor_scale
     E, N, dev = 3, 328, gpu_device
     ids, qa, sa, qb, sb, M_sum = _grouped_case(E, N, K, M_tok=300, topk=2, seed=K, dev=dev)
+    if not ue8m0:
+        sb = (sb * np.float32(1.37)).astype(np.float32)
     assert 160 * E <= M_sum < 160 * (E + 4)
-    A, sA, idt = to_fp8(qa, dev), torch.from_numpy(sa).to(dev), torch.from_numpy(ids).to(dev)
-    outs = []
-    for extra in (0, 4):
+    A, row, idt = to_fp8(qa, dev), torch.from_numpy(sa).to(dev), torch.from_numpy(ids).to(dev)
+    col = _alloc_colmajor_scale(M_sum, K // 128, dev)
+    col.copy_(row)
+    outs, glus = [], []
+    for sA, extra in ((row, 0), (col, 0), (col, 4)):
         B = to_fp8(np.concatenate([qb, qb[:1].repeat(extra, 0)]), dev)
         sB = torch.from_numpy(np.concatenate([sb, sb[:1].repeat(extra, 0)])).to(dev)
         C = torch.full((M_sum, N), 7.0, dtype=torch.bfloat16, device=dev)
-        _ops.m_grouped_gemm_nt_contiguous(A, sA, B, sB, C, idt, disable_ue8m0_cast=False)
+        _ops.m_grouped_gemm_nt_contiguous(A, sA, B, sB, C, idt, disable_ue8m0_cast=not ue8m0)
         outs.append(C)
+        q = torch.zeros(M_sum, 128, dtype=torch.float8_e4m3fn, device=dev)
+        s = _alloc_colmajor_scale(M_sum, 1, dev).zero_()
+        _ops.grouped_gemm_silu_quant(A, sA, B[:, :256].contiguous(), sB[:, :2].contiguous(), idt, not ue8m0, q, s)
+        glus.append((q, s))
     torch.cuda.synchronize()
     valid = ids >= 0
-    ref = oracle.grouped_gemm_nt_sample(qa, sa, qb, sb, ids)
-    assert_gemm_close(outs[0][torch.from_numpy(valid).to(dev)], ref[valid], f"four wavefronts, K={K}")
+    ref = oracle.grouped_gemm_nt_sample(qa, sa, qb, sb, ids, ue8m0=ue8m0)
+    assert_gemm_close(outs[0][torch.from_numpy(valid).to(dev)], ref[valid], f"K={K} ue8m0={ue8m0}")
     assert torch.all(outs[0][torch.from_numpy(~valid).to(dev)] == 7.0)
-    assert torch.equal(outs[0].view(torch.int16), outs[1].view(torch.int16))
+    for C, (q, s) in zip(outs[1:], glus[1:], strict=True):
+        assert torch.equal(outs[0].view(torch.int16), C.view(torch.int16))
+        assert torch.equal(glus[0][0].view(torch.uint8), q.view(torch.uint8)) and torch.equal(glus[0][1], s)
+    assert int((glus[0][0].view(torch.uint8) != 0).sum()) > 0
 
 
 def test_grouped_gemm_free_function_colmajor_scales(gpu_device):
