@@ -634,8 +634,13 @@ gemm_bs_kernel(const GemmArgs a) {
     // registers where there are few of them; the 256-row tiles add the row
     // part (uniform) to the first row's offset as each load is issued.
     // A and W loads go out in pairs that share one M0 write (dma_b128_pair);
-    // gathered rows may lie at offset 0, so they are loaded one by one.
-    constexpr bool kPairW = FM * FN < 8, kPairA = kPairW && !kSorted && kAInstr % 2 == 0;
+    // gathered rows may lie at offset 0, so they are loaded one by one; so are
+    // those of the 64x128 tiles of three stages, two workgroups of which share
+    // a CU: with pairs 64 x 57344 x 8192 took 84.0 us against 82.7, row-major
+    // scales as given 90.0 against 87.7, 64 x 40960 x 8192 85.8 against 82.9 (the
+    // bf16-input tiles keep pairs: 1 x 57344 x 8192 78.5 against 79.0).
+    constexpr bool kTwoWide = BM == 64 && BN == 128 && kStages == 3 && !kFuseA;
+    constexpr bool kPairW = FM * FN < 8 && !kTwoWide, kPairA = kPairW && !kSorted && kAInstr % 2 == 0;
     constexpr int kAUnits = kPairA ? kAInstr / 2 : kAInstr, kUnits = kScaleDma + kAUnits + kBInstr / (kPairW ? 2 : 1);
     constexpr bool kKeepOff = kAInstr + kBInstr <= 12 && FM * FN * kWaves <= 32;
     auto a_voff = [&](int i) -> int {
