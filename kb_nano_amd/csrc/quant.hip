@@ -67,7 +67,7 @@ constexpr int64_t kSmallSiluGroups = 32768;
 // 4-group blocks per wavefront per pass (per operand): the SiLU kernel runs
 // one workgroup per CU (its LDS table), so it takes more blocks per pass to
 // keep as many bytes in flight (measured at cfg2: 4 -> 129 us, 2 -> 132 us,
-// 5..8 -> 136-140 us; the quant kernel is best at 2).  The row-skipping
+// 5..8 -> 136-140 us); the quant of fp16 and fp32 inputs takes 2.  The row-skipping
 // mode is best at 4 as well (cfg4 layout: 88 us against 90-92 us at 6 and 8).
 template <bool kSilu>
 constexpr int kUnrollOf = kSilu ? 4 : 2;
